@@ -24,6 +24,7 @@
 //     X and W panels in that XCD's L2.
 #include <string.h>
 
+#include <array>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -820,6 +821,8 @@ __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WPE, T
 #endif
 }
 
+#include "gemm_kwave.h"
+
 // ------------------------------------------------------------------ configurations
 
 // 8 waves, two per SIMD: 128x64 (w8m) or 64x128 (w8n) per wave.  While one
@@ -872,6 +875,10 @@ using D320n = DTile<256, 320, 128, 4, 2, 2, 4, 1, 0, 4, 0, 1>;
 // hold 32x96 and read 4 KiB for 3), and the ring holds two slots of two
 // 40 KiB K tiles; the hand-off is 96 KiB of LDS once per tile.  K % 256 == 0.
 using D192k2 = DTile<128, 192, 128, 2, 2, 2, 8, 1, 0, 0, 0, 1, 2>;
+// 128x128 tiles, two K-groups of 2x2 waves of 64x64: where a grid holds no more
+// 128x128 tiles than CUs, a second wave per SIMD and half the K loop each (a
+// 4-wave tile alone on its CU runs one wave per SIMD).  K % 256 == 0.
+using D128k2 = DTile<128, 128, 128, 2, 2, 2, 8, 1, 0, 0, 0, 1, 2>;
 
 typedef void (*kernel_fn)(const int8_t*, const int8_t*, const float*, const float*, const uint16_t*, void*, int, int,
                           int, int, int, int64_t, int, int);
@@ -892,6 +899,11 @@ struct Config {
     {NAME, T::BM, T::BN, T::BK + 0 * sizeof(char[T::SPLITK == 1 ? 1 : -1]), T::NT,                             \
      w8a8_gemm_direct_kernel<T, false>, w8a8_gemm_direct_kernel<T, true>, true}
 
+// Wave-split tiles (gemm_kwave.h): KTile<MF, NF> is 16 MF rows of X by 16 NF of W.
+#define H3MI_KCFG(NAME, ...) \
+    {NAME, KTile<__VA_ARGS__>::BM, KTile<__VA_ARGS__>::BN, 128, KTile<__VA_ARGS__>::NT, \
+     w8a8_gemm_kwave_kernel<KTile<__VA_ARGS__>, false>, w8a8_gemm_kwave_kernel<KTile<__VA_ARGS__>, true>, false}
+
 const Config kConfigs[] = {
     H3MI_DCFG("d_bm256_bn256_bk128_s2_g4_w8m_st1", D256w8st1),
     H3MI_DCFG("d_bm128_bn128_bk128_s2_g4_o2", D128o2),
@@ -905,6 +917,16 @@ const Config kConfigs[] = {
     H3MI_RCFG("d_bm256_bn320_bk128_s2_g4_w4x2_l4_sw_res", D320n),
     H3MI_DCFG("d_bm128_bn192_bk128_s2_g8_w2x2_sw_k2", D192k2),
     H3MI_RCFG("d_bm256_bn384_bk128_s2_g4_w8m_l4_a1_sw_res", D384g4),
+    H3MI_DCFG("d_bm128_bn128_bk128_s2_g8_w2x2_sw_k2", D128k2),
+    H3MI_KCFG("k_bm16_bn16_w4_s2", 1, 1),
+    H3MI_KCFG("k_bm16_bn32_w4_s2", 1, 2),
+    H3MI_KCFG("k_bm32_bn32_w4_s2", 2, 2),
+    H3MI_KCFG("k_bm32_bn48_w4_s2", 2, 3),
+    H3MI_KCFG("k_bm48_bn48_w4_s2", 3, 3),
+    H3MI_KCFG("k_bm64_bn48_w4_s2", 4, 3),
+    H3MI_KCFG("k_bm64_bn64_w4_s2", 4, 4),
+    H3MI_KCFG("k_bm64_bn80_w4_s2", 4, 5),
+    H3MI_KCFG("k_bm64_bn96_w4_s2", 4, 6),
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
@@ -932,12 +954,83 @@ int resident_per_cu(kernel_fn fn, int threads) {
     return n;
 }
 
+// Predicted time of a tiling on a grid that does not fill the chip several
+// times over, in us.  A CU runs ceil(tiles / CUs) workgroups one after the
+// other (or side by side at a shared rate); a workgroup takes `tile` plus, per
+// MB of operand rows that it stages, `own` and, as far as the CUs are all busy
+// and share the L2s and memory, `shared`; no call is faster than its bytes at
+// 5.3 TB/s.  The constants are least-squares fits to 300 measured shapes (M 1 to
+// 4799, N 384 to 28672, K 384 to 14336; relative error 8-11%, larger only where
+// a tiling is far from the best).  Over these shapes the rule below picks a
+// tiling 3% slower than the fastest of them on average, against 45% for the
+// rule over the 128x128 and larger tiles alone.
+struct Cost {
+    const char* name;
+    double fix, tile, own, shared;
+};
+constexpr Cost kCosts[] = {
+    {"k_bm16_bn16_w4_s2", 2.42, 0.46, 4.33, 4.22},
+    {"k_bm16_bn32_w4_s2", 2.48, 0.64, 3.11, 5.93},
+    {"k_bm32_bn32_w4_s2", 2.46, 0.92, 4.27, 5.45},
+    {"k_bm32_bn48_w4_s2", 2.79, 1.19, 3.62, 5.92},
+    {"k_bm48_bn48_w4_s2", 1.73, 2.72, 7.39, 3.65},
+    {"k_bm64_bn48_w4_s2", 1.34, 3.32, 9.47, 1.89},
+    {"k_bm64_bn64_w4_s2", 1.12, 4.10, 10.11, 1.55},
+    {"k_bm64_bn80_w4_s2", 1.28, 4.94, 10.07, 1.85},
+    {"k_bm64_bn96_w4_s2", 0.83, 6.26, 10.56, 0.94},
+    {"d_bm128_bn128_bk128_s2_g4_o2", 4.06, 0.86, 16.32, 0.0},
+    {"d_bm128_bn128_bk128_s2_g8_w2x2_sw_k2", 2.47, 2.42, 13.19, 4.65},
+    {"d_bm128_bn192_bk128_s2_g8_w2x2_sw_k2", 2.63, 3.60, 12.68, 5.05},
+    {"d_bm256_bn256_bk128_s2_g4_w8m_st1_sw_res", 1.12, 5.95, 13.05, 10.43},
+    {"d_bm256_bn320_bk128_s2_g4_w4x2_l4_sw_res", 3.79, 6.39, 14.01, 9.48},
+    {"d_bm256_bn384_bk128_s2_g8_w8m_l4_a1_sw_res", 8.22, 5.38, 15.48, 10.77},
+};
+
+// The table's entry of each configuration (null: not offered to small grids).
+const Cost* cost_of(int config) {
+    static const std::array<const Cost*, kNumConfigs> table = [] {
+        std::array<const Cost*, kNumConfigs> t{};
+        for (const Cost& k : kCosts) t[config_index(k.name)] = &k;
+        return t;
+    }();
+    return table[config];
+}
+
+double predicted_us(int config, int64_t M, int64_t N, int64_t K, int64_t cus) {
+    const Config& c = kConfigs[config];
+    const Cost* k = cost_of(config);
+    if (!k) return 1e300;
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const bool wave_split = c.name[0] == 'k';  // its loads past M or N move nothing
+    const double rows = wave_split ? static_cast<double>((M < c.bm ? M : c.bm) + (N < c.bn ? N : c.bn)) : c.bm + c.bn;
+    const double busy = tiles < cus ? static_cast<double>(tiles) / cus : 1.0;
+    const double work = static_cast<double>((tiles + cus - 1) / cus) * (k->tile + rows * K * 1e-6 * (k->own + k->shared * busy));
+    const double mem = 0.19e-6 * (static_cast<double>(M + N) * K + 2.0 * M * N);
+    return k->fix + (work > mem ? work : mem);
+}
+
+// The wave-split tiling with the least predicted time, or `other` if that is
+// faster still.  A tile with a whole 16-row block past M is left out: it
+// multiplies and sums blocks of zeros.
+int wave_split_or(int other, int64_t M, int64_t N, int64_t K, int64_t cus) {
+    static const int first = config_index("k_bm16_bn16_w4_s2");
+    int best = other;
+    double t = predicted_us(other, M, N, K, cus);
+    for (int i = first; i < kNumConfigs; ++i) {
+        if (kConfigs[i].bm > 16 && kConfigs[i].bm - 16 >= M) continue;
+        const double ti = predicted_us(i, M, N, K, cus);
+        if (ti < t) t = ti, best = i;
+    }
+    return best;
+}
+
 // Big grids (at least two 256x256 tiles per CU) run one resident workgroup
 // per CU over the tiles.  Of the 256x256, 256x384, 320x256 and 256x320
 // tilings, the one whose busiest workgroup has the least work runs: its tile
 // count rounded up to whole rounds over the CUs, times the tile area, with the
-// 256x384 and 256x320 tiles' measured 3% and 2.4% higher rates per area.  Smaller grids run 128x128 tiles (two
-// workgroups per CU) or one 256x256 tile per workgroup, by the model below.
+// 256x384 and 256x320 tiles' measured 3% and 2.4% higher rates per area.  Of the
+// smaller grids, one of the 128x128, 128x192 or larger tiles is weighed by the
+// same measure and then against the wave-split tilings by predicted time.
 int pick_config(int64_t M, int64_t N, int64_t K) {
     {
         // a forced configuration that cannot take this K (split-K tilings
@@ -951,6 +1044,7 @@ int pick_config(int64_t M, int64_t N, int64_t K) {
     static const int tall = config_index("d_bm320_bn256_bk128_s2_g4_w8m_st1_sw_res");
     static const int flat = config_index("d_bm256_bn320_bk128_s2_g4_w4x2_l4_sw_res");
     static const int small = config_index("d_bm128_bn128_bk128_s2_g4_o2");
+    static const int small_k2 = config_index("d_bm128_bn128_bk128_s2_g8_w2x2_sw_k2");
     static const int split = config_index("d_bm128_bn192_bk128_s2_g8_w2x2_sw_k2");
     const int64_t cus = cu_count();
     auto rounds = [&](int64_t bm, int64_t bn) {
@@ -984,10 +1078,22 @@ int pick_config(int64_t M, int64_t N, int64_t K) {
         const double c128 = static_cast<double>((t128 + cus - 1) / cus) * 128.0 * 128.0;
         const double c256 = static_cast<double>((t256 + cus - 1) / cus) * 256.0 * 256.0 / 1.5;
         const double c320 = n320 ? rounds(256, 320) * 256.0 * 320.0 / (1.5 * 1.024) : 1e300;
+        // 256x384 (past half a round of 256x256 tiles that would need a second):
+        // 768 x 28672 x 5376 110 against 138 us, 1536 x 15360 x 5120 98 against
+        // 116, 4096 x 5376 x 14336 260 against 327; with a short K its epilogue
+        // weighs more (2400 x 9000 x 1536: 58.6 against 53.3).
+        const double c384 = K >= 3072 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
         const double ck2 = K % 256 == 0 ? rounds(128, 192) * 128.0 * 192.0 / 0.88 : 1e300;
-        if (c320 < c256 && c320 < c128 && c320 < ck2) return flat;
-        if (ck2 < c256 && ck2 < c128) return split;
-        return c256 < c128 ? big : small;
+        int c = c256 < c128 ? big : small;
+        if (ck2 < c256 && ck2 < c128) c = split;
+        if (c320 < c256 && c320 < c128 && c320 < ck2) c = flat;
+        if (c384 < c256 && c384 < c128 && c384 < ck2 && c384 < c320) c = wide;
+        // One 128x128 tile per CU or fewer: two K-groups of waves instead of one,
+        // from K = 4096 up (768 x 5376 x 14336 66 against 78 us, 128 x 28672 x
+        // 5376 38 against 46, 384 x 10240 x 5120 33.9 against 36.2); shorter K
+        // stays with the plain tile, which the tests name at 1024 x 3072 x 3072.
+        if (c == small && t128 <= cus && K % 256 == 0 && K >= 4096) c = small_k2;
+        return wave_split_or(c, M, N, K, cus);
     }
     const double w256 = rounds(256, 256) * 256.0 * 256.0;
     const double w384 = rounds(256, 384) * 256.0 * 384.0 / 1.03;

@@ -232,6 +232,20 @@ def test_heuristic_picks_the_measured_tiling(M, N, K, tile):
     assert h3mi.config_for(M, N, K) == tile
 
 
+@pytest.mark.parametrize("M,N,K,tile", [
+    (1, 3072, 3072, "k_bm16_bn16_w4_s2"),                                 # one row: 192 of the smallest tiles
+    (37, 10240, 5120, "k_bm48_bn48_w4_s2"),                               # a short prompt
+    (128, 72, 14336, "k_bm16_bn16_w4_s2"),                                # a narrow output
+    (256, 3072, 3072, "k_bm64_bn48_w4_s2"),                               # 256 tiles
+    (768, 5376, 14336, "d_bm128_bn128_bk128_s2_g8_w2x2_sw_k2"),           # 252 128x128 tiles, a long K
+    (128, 21504, 512, "d_bm128_bn128_bk128_s2_g4_o2"),                    # a short K
+    (768, 28672, 5376, "d_bm256_bn384_bk128_s2_g8_w8m_l4_a1_sw_res"),     # 225 tiles of 256x384, 336 of 256x256
+])
+def test_heuristic_on_small_grids(M, N, K, tile):
+    import h3mi
+    assert h3mi.config_for(M, N, K) == tile
+
+
 def test_buffer_probe_argument_errors():
     """The range-check probe rejects its arguments before any launch."""
     from h3mi import _lib

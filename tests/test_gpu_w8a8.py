@@ -211,7 +211,43 @@ def test_every_tile_config_matches(M, N, K):
         h.set_config("auto")
 
 
-SPLITK = ["d_bm128_bn192_bk128_s2_g8_w2x2_sw_k2"]
+@pytest.mark.parametrize("M,N,K", [(1, 4, 128), (15, 20, 384), (16, 16, 512), (17, 36, 640), (49, 100, 1152),
+                                   (65, 52, 1024), (97, 196, 2176), (37, 1028, 5120)])
+def test_wave_split_tilings_match_oracle(M, N, K):
+    """Wave-split tilings: one to 40 K slices of 128 bytes over 4 waves of two
+    slots each (fewer slices than waves, waves with no slice, odd counts), edges
+    of the 16-row blocks and of whole tiles, single rows and columns."""
+    h = _h3mi()
+    g = np.random.default_rng(M * 11 + N + K)
+    xq = g.integers(-127, 128, (M, K), dtype=np.int8)
+    w = g.integers(-127, 128, (N, K), dtype=np.int8)
+    xs = (0.05 * g.random((M, 1))).astype(np.float32)
+    ws = (1e-3 + 9e-3 * g.random(N)).astype(np.float32)
+    bias = O.f32_to_bf16_bits((0.02 * g.standard_normal((1, N))).astype(np.float32))[0]
+    acc = (xq.astype(np.float64) @ w.astype(np.float64).T).astype(np.int32)
+    # operands inside larger buffers whose padding would change the sums if read
+    xp, wp = torch.full((M + 1, K + 16), 99, dtype=torch.int8), torch.full((N + 1, K + 48), 77, dtype=torch.int8)
+    xp[:M, :K], wp[:N, :K] = torch.from_numpy(xq), torch.from_numpy(w)
+    xd, wd, xsd, wsd, bd = (t.cuda() for t in (xp, wp, torch.from_numpy(xs), torch.from_numpy(ws), from_bits(bias)))
+    from h3mi._lib import check, lib, ptr, stream_of
+    names = [nm for nm in h.list_configs() if nm.startswith("k_")]
+    assert len(names) >= 2
+    try:
+        for nm in names:
+            print(f"[wave-split] {nm} M={M} N={N} K={K}", flush=True)
+            h.set_config(nm)
+            out = torch.full((M, N + 4), 7, dtype=torch.bfloat16, device="cuda")
+            check(lib.h3mi_w8a8_gemm_bf16(ptr(xd), ptr(wd), ptr(xsd), ptr(wsd), ptr(bd), ptr(out), M, N, K, K + 16,
+                                          K + 48, N + 4, stream_of(xd)))
+            assert np.array_equal(bits(out[:, :N]), O.epilogue_bf16(acc, xs, ws, bias)), nm
+            assert bool((out[:, N:] == 7).all()), nm
+            assert np.array_equal(h.int8_mm_i32(torch.from_numpy(xq).cuda(), torch.from_numpy(w).cuda()).cpu().numpy(),
+                                  acc), nm
+    finally:
+        h.set_config("auto")
+
+
+SPLITK = ["d_bm128_bn192_bk128_s2_g8_w2x2_sw_k2", "d_bm128_bn128_bk128_s2_g8_w2x2_sw_k2"]
 
 
 @pytest.mark.parametrize("name", SPLITK)
