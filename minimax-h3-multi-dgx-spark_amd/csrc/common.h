@@ -172,7 +172,7 @@ __device__ __forceinline__ bool quot_fast(float sc, float r) {
     return sc >= 0x1p-126f && sc <= 0x1p+126f && r <= 0x1p+126f;
 }
 
-// Per-token int8 quantization of 8 elements whose values are bf16 numbers, as
+// Per-token int8 quantization of 4 or 8 elements whose values are bf16 numbers, as
 // the per-token quantizer and the norm -> quantizer fusion have them (|e| <=
 // amax, amax a bf16 value, sc = fl(amax / 127), r = fl(1 / sc)):
 // clamp(rne(fl(e / sc)), -127, 127), with no residual test and no branch per
@@ -194,34 +194,33 @@ __device__ __forceinline__ bool quot_exact(float sc, float r) {
     return sc >= 0x1p-100f && sc <= 0x1p+126f && r <= 0x1p+126f;
 }
 
-__device__ __forceinline__ uint2 quant8b(const float (&e)[8], float sc, float r, bool exact) {
+__device__ __forceinline__ uint32_t quant4b(float e0, float e1, float e2, float e3, float sc, float r, bool exact) {
 #pragma clang fp contract(off)
-    float n[8];
+    const float e[4] = {e0, e1, e2, e3};
+    float n[4];
     if (exact) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < 4; ++j) {
             const float q0 = e[j] * r;
             const float rem = __builtin_fmaf(-q0, sc, e[j]);
             n[j] = __builtin_fmaf(rem, r, q0);
         }
         // the magic add writes its low byte straight into place
         const float mg = kQuantMagic;
-        uint32_t lo, hi;
-        add_low_byte<0>(lo, n[0], mg);
-        add_low_byte<1>(lo, n[1], mg);
-        add_low_byte<2>(lo, n[2], mg);
-        add_low_byte<3>(lo, n[3], mg);
-        add_low_byte<0>(hi, n[4], mg);
-        add_low_byte<1>(hi, n[5], mg);
-        add_low_byte<2>(hi, n[6], mg);
-        add_low_byte<3>(hi, n[7], mg);
-        return make_uint2(lo, hi);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) n[j] = fminf(fmaxf(rintf(e[j] / sc), -127.0f), 127.0f) + kQuantMagic;
+        uint32_t p;
+        add_low_byte<0>(p, n[0], mg);
+        add_low_byte<1>(p, n[1], mg);
+        add_low_byte<2>(p, n[2], mg);
+        add_low_byte<3>(p, n[3], mg);
+        return p;
     }
-    return make_uint2(pack_low_bytes(__float_as_uint(n[0]), __float_as_uint(n[1]), __float_as_uint(n[2]), __float_as_uint(n[3])),
-                      pack_low_bytes(__float_as_uint(n[4]), __float_as_uint(n[5]), __float_as_uint(n[6]), __float_as_uint(n[7])));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) n[j] = fminf(fmaxf(rintf(e[j] / sc), -127.0f), 127.0f) + kQuantMagic;
+    return pack_low_bytes(__float_as_uint(n[0]), __float_as_uint(n[1]), __float_as_uint(n[2]), __float_as_uint(n[3]));
+}
+
+__device__ __forceinline__ uint2 quant8b(const float (&e)[8], float sc, float r, bool exact) {
+    return make_uint2(quant4b(e[0], e[1], e[2], e[3], sc, r, exact), quant4b(e[4], e[5], e[6], e[7], sc, r, exact));
 }
 
 // quant8b of 8 packed bf16 values (2 per word).

@@ -1273,6 +1273,174 @@ __global__ __launch_bounds__(256) void gate_norm_split_kernel(
     else run(std::true_type{});
 }
 
+// ------------------------------------------------------------------ one row per workgroup, not persistent
+
+// For calls whose tensors the caches still hold or whose rows are few per CU,
+// and for tables of several rows (rows_suit below).  There the row streams'
+// set-up -- counting the table rows, copying them to LDS as fp32, a barrier
+// each -- and the one or two rows that a wave has in flight are most of the
+// call, and a row whose table row is not the staged one reads its tables late.
+// A workgroup of 256 threads takes one row in the default order's own layout
+// (gate_norm_split_kernel) and every load of the row, the tables' included,
+// goes out at once; the tables come from L2.  What bounds it: at few rows the
+// chain of one load latency, the reduction and the stores (4 us with the
+// launch), then the caches' and memory's rate with 5-8 rows in flight per CU.
+// At N = 5376, us before -> after: norm_mod 512 rows 9.8 -> 4.9, 2401 17.3 ->
+// 13.4; norm_mod_q 512 10.8 -> 5.9, 2401 20.2 -> 14.4; gate_norm_mod_ 512 11.0
+// -> 6.9, 2401 26.4 -> 22.0; gate_norm_mod_q_ 512 14.0 -> 8.0, 2401 32.9 ->
+// 21.7 (graph replays).  Loads through the cache, stores non-temporal: cached
+// stores 2-15% slower, non-temporal loads 15-30%.  QUANT as in norm_stream_rows.
+template <int IT, bool GATE, int QUANT>
+__global__ __launch_bounds__(256) void norm_row_kernel(
+    uint16_t* __restrict__ x, const uint16_t* __restrict__ o, const uint16_t* __restrict__ g,
+    const uint16_t* __restrict__ w, const int32_t* __restrict__ ridx, const uint16_t* __restrict__ s1,
+    const uint16_t* __restrict__ sh, uint16_t* __restrict__ h, int N, int R, float eps, int rsq_mode,
+    float* __restrict__ row_var, float* __restrict__ row_rstd, int8_t* __restrict__ q, float* __restrict__ qs) {
+    __shared__ float red[8];  // the warp totals, then the waves' maxima
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int64_t row = blockIdx.x;
+    auto load = [&](v2u_t (&d)[IT], __amdgpu_buffer_rsrc_t rs) {
+#pragma unroll
+        for (int it = 0; it < IT; ++it)
+            d[it] = __builtin_bit_cast(v2u_t, __builtin_amdgcn_raw_buffer_load_b64(rs, (it * 1024 + 4 * t) * 2, 0, 0));
+    };
+    auto store = [&](__amdgpu_buffer_rsrc_t rs, int it, v2u_t v) {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i_t, v), rs, (it * 1024 + 4 * t) * 2, 0, 2);
+    };
+    // elements past N read as zero and are not stored
+    const __amdgpu_buffer_rsrc_t xr = span_rsrc(x + row * N, N * 2);
+    v2u_t X[IT], O[GATE ? IT : 1], G[GATE ? IT : 1], W[IT], S1[IT], SH[IT];
+    load(X, xr);
+    if constexpr (GATE) load(O, span_rsrc(o + row * N, N * 2));
+    const int r = ridx[row];
+    if (r < 0 || r >= R) return;  // uniform: the row is left unwritten
+    const int64_t tab = static_cast<int64_t>(r) * N;
+    if constexpr (GATE) load(G, span_rsrc(g + tab, N * 2));
+    load(W, span_rsrc(w, N * 2));
+    load(S1, span_rsrc(s1 + tab, N * 2));
+    load(SH, span_rsrc(sh + tab, N * 2));
+    __builtin_amdgcn_sched_barrier(0);  // every load is out before the row is summed
+
+    float acc = 0.0f;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        if constexpr (GATE) X[it] = gate4f(X[it], O[it], unpack4(G[it]));
+        const F4 f = unpack4(X[it]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc += f.f[j] * f.f[j];
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d /= 2) acc += __shfl_down(acc, d, 64);
+    if (lane == 0) red[wv] = acc;
+    wait_lgkm0();
+    wg_barrier();
+    const float tot = (red[0] + red[2]) + (red[1] + red[3]);
+    const float var = tot / static_cast<float>(N) + eps;
+    const float rstd = rsqrt_mode(var, rsq_mode);
+    if (t == 0) {
+        if (row_var) row_var[row] = var;
+        if (row_rstd) row_rstd[row] = rstd;
+    }
+    const __amdgpu_buffer_rsrc_t hr = span_rsrc(h + (QUANT == 1 ? 0 : row * N), QUANT == 1 ? 0 : N * 2);
+    F4 hf[QUANT ? IT : 1];
+    float amax = 0.0f;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        if constexpr (GATE) store(xr, it, X[it]);
+        const v2u_t hv = mod4f(unpack4(X[it]), unpack4(W[it]), unpack4(S1[it]), unpack4(SH[it]), rstd);
+        if constexpr (QUANT != 1) store(hr, it, hv);
+        if constexpr (QUANT != 0) {
+            hf[it] = unpack4(hv);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) amax = fmaxf(amax, fabsf(hf[it].f[j]));
+        }
+    }
+    if constexpr (QUANT != 0) {
+        amax = wave_max(amax);
+        if (lane == 0) red[4 + wv] = amax;
+        wait_lgkm0();
+        wg_barrier();
+        amax = wave_uniform(fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7])));
+        const float sc = amax / 127.0f;
+        if (t == 0) qs[row] = sc;
+        const float rc = 1.0f / sc;
+        const bool exact = quot_exact(sc, rc);  // h is bf16, so quant4b applies
+        const __amdgpu_buffer_rsrc_t qr = span_bytes(q + row * N, N);
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const F4& e = hf[it];
+            const uint32_t p = sc != 0.0f ? quant4b(e.f[0], e.f[1], e.f[2], e.f[3], sc, rc, exact) : 0u;
+            // a cached store: the GEMM reads q next
+            __builtin_amdgcn_raw_buffer_store_b32(p, qr, it * 1024 + 4 * t, 0, 0);
+        }
+    }
+}
+
+// gate_ the same way, 16 bytes per thread and load: at N = 5376 512 rows 9.0 ->
+// 4.4 us, 2401 19.0 -> 13.2; at N = 1024 38400 rows 70.7 -> 47.2; 9600 x 5376 over
+// five table rows 104.7 -> 55.6.
+template <int IT>
+__global__ __launch_bounds__(256) void gate_row_kernel(uint16_t* __restrict__ x, const uint16_t* __restrict__ o,
+                                                       const uint16_t* __restrict__ g,
+                                                       const int32_t* __restrict__ ridx, int N, int R) {
+    const int t = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    const __amdgpu_buffer_rsrc_t xr = span_rsrc(x + row * N, N * 2), orr = span_rsrc(o + row * N, N * 2);
+    v4u_t X[IT], O[IT], G[IT];
+    auto load = [&](v4u_t (&d)[IT], __amdgpu_buffer_rsrc_t rs) {
+#pragma unroll
+        for (int it = 0; it < IT; ++it)
+            d[it] = __builtin_bit_cast(v4u_t, __builtin_amdgcn_raw_buffer_load_b128(rs, (it * 2048 + 8 * t) * 2, 0, 0));
+    };
+    load(X, xr);
+    load(O, orr);
+    const int r = ridx[row];
+    if (r < 0 || r >= R) return;  // uniform: the row is left as it is
+    load(G, span_rsrc(g + static_cast<int64_t>(r) * N, N * 2));
+#pragma unroll
+    for (int it = 0; it < IT; ++it) store_row16(xr, it * 2048 + 8 * t, gate8(X[it], O[it], G[it]));
+}
+
+// Whether a call of S rows runs the one-row-per-workgroup kernels (gate_ has its
+// own line).  With one table row the streams win once the tensors come from
+// memory (with inputs rotated past the caches the two meet at about 16 Mi
+// elements, 24 Mi with the quantizer, whose streams have less of a row in
+// flight), and, in rows narrower than a workgroup, past about 20 rows per CU
+// (at N = 512 9600 rows: norm_mod 12.5 against 14.0 us, norm_mod_q 16.8 against
+// 14.6); gate_norm_mod_'s own stream, a workgroup per row and CU, is behind at
+// any S for N = 1024 to 2048 (38400 x 1024: 106.7 against 67.9).  With several
+// table rows a stream reads most rows' tables from L2 after their x, and the
+// lines move: 38400 x 5376 over five, gate_norm_mod_ 470 against 323 us,
+// gate_norm_mod_q_ 380 against 325, norm_mod 209 against 201, but norm_mod_q 170
+// against 188; over two, gate_norm_mod_ 361 against 325, gate_norm_mod_q_ 175
+// against 172 at 19200 rows and 303 against 319 at 38400, norm_mod 30.4 against
+// 28.7 at 4800 and 52 against 57 at 9600.
+bool rows_suit(bool gate, bool quant, int64_t S, int64_t N, int64_t R) {
+    const int64_t mi = S * N >> 20;
+    if (R > 1) {
+        if (gate) return !quant || R > 3 || mi < 100;
+        return quant ? mi < 32 : R > 3 || mi < 24;
+    }
+    if (gate && !quant && N >= 1024 && N <= 2048) return true;
+    return S <= 5120 && mi < (quant ? 24 : 16);
+}
+
+template <bool GATE, int QUANT>
+int launch_rows(uint16_t* x, const uint16_t* o, const uint16_t* g, const uint16_t* w, const int32_t* ridx,
+                const uint16_t* s1, const uint16_t* sh, uint16_t* h, int64_t S, int N, int R, float eps, int rsq,
+                float* var, float* rstd, int8_t* q, float* qs, hipStream_t st, const char* name) {
+    const int it = (N + 1023) / 1024;
+    const dim3 grid(static_cast<unsigned>(S)), block(256);
+#define H3MI_ROW_LAUNCH(I)                                                                                            \
+    if (it == I)                                                                                                      \
+        hipLaunchKernelGGL((norm_row_kernel<I, GATE, QUANT>), grid, block, 0, st, x, o, g, w, ridx, s1, sh, h, N, R,  \
+                           eps, rsq, var, rstd, q, qs);
+    H3MI_ROW_LAUNCH(1) H3MI_ROW_LAUNCH(2) H3MI_ROW_LAUNCH(3) H3MI_ROW_LAUNCH(4)
+    H3MI_ROW_LAUNCH(5) H3MI_ROW_LAUNCH(6) H3MI_ROW_LAUNCH(7) H3MI_ROW_LAUNCH(8)
+#undef H3MI_ROW_LAUNCH
+    return check_launch(name);
+}
+
 template <int NUMX, int WARP, bool GATE>
 int launch_order(uint16_t* x, const uint16_t* o, const uint16_t* g, const uint16_t* w, const int32_t* ridx,
                  const uint16_t* s1, const uint16_t* sh, uint16_t* h, int64_t S, int N, int R, float eps,
@@ -1280,6 +1448,9 @@ int launch_order(uint16_t* x, const uint16_t* o, const uint16_t* g, const uint16
     // Persistent row stream for N <= 8192 in the product order; the reference
     // order (a parity mode) keeps the kernels below.
     const int ch = (NUMX == 256 && WARP == 64) ? stream_ch(N) : 0;
+    if (ch > 0 && rows_suit(GATE, false, S, N, R))
+        return launch_rows<GATE, 0>(x, o, g, w, ridx, s1, sh, h, S, N, R, eps, rsq, var, rstd, nullptr, nullptr, st,
+                                    GATE ? "gate_norm_mod" : "norm_mod");
     if (GATE && ch > 0 && N >= 1024 && (N % 1024 == 0 || N % 1024 == 256)) {
         const int it = N / 1024, tail = N % 1024 ? 1 : 0;
         const size_t slds = static_cast<size_t>(4 * (it + tail) * 1024 + 8) * sizeof(float);
@@ -1405,6 +1576,11 @@ int norm_quant_entry(uint16_t* x, const uint16_t* o, const uint16_t* g, const ui
     // With the gate (7 bytes per element) one workgroup per CU stays best.
     const dim3 grid(stream_grid(S, GATE ? 1 : 2)), block(256);
     hipStream_t st = as_stream(stream);
+    if (rows_suit(GATE, true, S, N, R))
+        return h ? launch_rows<GATE, 2>(x, o, g, w, ridx, s1, sh, h, S, (int)N, (int)R, eps, H3MI_RSQRT_HW, nullptr,
+                                        nullptr, q, qs, st, name)
+                 : launch_rows<GATE, 1>(x, o, g, w, ridx, s1, sh, h, S, (int)N, (int)R, eps, H3MI_RSQRT_HW, nullptr,
+                                        nullptr, q, qs, st, name);
 #define H3MI_QUANT_LAUNCH(C)                                                                                          \
     if (ch == C) {                                                                                                    \
         if (h)                                                                                                        \
@@ -1486,6 +1662,19 @@ extern "C" int h3mi_gate_bf16(uint16_t* x, const uint16_t* o, const uint16_t* g,
     if (overlap(o, xb, x, xb)) return fail(H3MI_EALIAS, "gate: o overlaps x");
     if (overlap(g, static_cast<size_t>(R) * N * 2, x, xb)) return fail(H3MI_EALIAS, "gate: g overlaps x");
     const int ch = stream_ch(static_cast<int>(N));
+    // One row per workgroup, except over one table row for wide rows that come
+    // from memory: 19200 x 5376 107 against 102 us for the stream, 4800 x 5376 25
+    // against 30, 19200 x 3072 63 against 75.
+    if (ch > 0 && (R > 1 || N <= 4096 || S * N <= int64_t{40} << 20)) {
+        const int it = static_cast<int>((N + 2047) / 2048);
+        const dim3 grid(static_cast<unsigned>(S)), block(256);
+#define H3MI_GATE_ROW_LAUNCH(I)                                                                               \
+    if (it == I)                                                                                              \
+        hipLaunchKernelGGL((gate_row_kernel<I>), grid, block, 0, as_stream(stream), x, o, g, ridx, (int)N, (int)R);
+        H3MI_GATE_ROW_LAUNCH(1) H3MI_GATE_ROW_LAUNCH(2) H3MI_GATE_ROW_LAUNCH(3) H3MI_GATE_ROW_LAUNCH(4)
+#undef H3MI_GATE_ROW_LAUNCH
+        return check_launch("gate");
+    }
     if (ch > 0) {  // persistent row stream, N <= 8192
         // One wave per workgroup and per CU: it has 20 KiB of x and o in
         // flight, and fewer bytes in flight stream faster here.  Measured at

@@ -1,0 +1,56 @@
+"""The fused norms' two routes give the same bytes: a call of many rows (the
+row streams) against the same rows in calls of few (one row per workgroup,
+which the other norm tests hold against the oracle), on either side of the
+lines between them, with rows whose table index is out of range (left
+unwritten) when the table has several rows."""
+import numpy as np
+import pytest
+import torch
+
+from util import norm_inputs
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-6
+
+
+def _calls(h, x, w, s1, sh, g, o, ridx):
+    """Every norm of the rows: outputs start from a fill, so unwritten rows show."""
+    s, n = x.shape
+    new = lambda: torch.full_like(x, 3)
+    outs = []
+    hx = new()
+    _, var, rstd = h.norm_mod_ex(x, w, EPS, ridx, s1, sh, stats=True, h=hx)
+    ok = (ridx >= 0) & (ridx < s1.shape[0])
+    outs += [hx, var[ok], rstd[ok]]
+    xa, ha = x.clone(), new()
+    h.gate_norm_mod_ex(xa, o, g, w, EPS, ridx, s1, sh, h=ha)
+    outs += [xa, ha, h.gate_(x.clone(), o, g, ridx)]
+    if n % 8 == 0 and n <= 8192:
+        for want in (False, True):
+            outs += [t[ok] for t in h.norm_mod_q(x, w, EPS, ridx, s1, sh, want_h=want)]
+            xb = x.clone()
+            outs += [xb] + [t[ok] for t in h.gate_norm_mod_q_(xb, o, g, w, EPS, ridx, s1, sh, want_h=want)]
+    return outs
+
+
+@pytest.mark.parametrize("S,N,R", [(5125, 8, 1), (5125, 520, 1), (5121, 1032, 1), (5121, 2048, 1), (5600, 3072, 1),
+                                   (5000, 5376, 1), (8200, 5120, 1), (3100, 8192, 1), (4800, 5376, 2), (6500, 5376, 2),
+                                   (1500, 264, 5), (9800, 3584, 3)])
+def test_streams_and_rows_agree(S, N, R):
+    import h3mi as h
+    x, w, s1, sh, g, o, ridx = norm_inputs(S, N, R, seed=S + N, stress=True)
+    if R > 1:
+        ridx = (torch.arange(S) * R // S).to(torch.int32)
+        ridx[S // 2], ridx[S - 1] = -1, R
+    x, w, s1, sh, g, o, ridx = (t.cuda() for t in (x, w, s1, sh, g, o, ridx))
+    print(f"[routes] S={S} N={N} R={R}", flush=True)
+    whole = _calls(h, x, w, s1, sh, g, o, ridx)
+    step = 700
+    parts = [_calls(h, x[i:i + step].contiguous(), w, s1, sh, g, o[i:i + step].contiguous(), ridx[i:i + step].contiguous())
+             for i in range(0, S, step)]
+    for k, t in enumerate(whole):
+        ref = torch.cat([p[k] for p in parts])
+        assert torch.equal(t.contiguous().view(torch.uint8), ref.contiguous().view(torch.uint8)), k
+    if R > 1:  # out-of-range rows keep the fill and x
+        assert bool((whole[0][S // 2] == 3).all()) and torch.equal(whole[5][S // 2], x[S // 2])
