@@ -34,98 +34,130 @@ namespace {
 
 typedef uint32_t v4u_t __attribute__((ext_vector_type(4)));
 
+// n / d for n < 2^31 and d >= 2: (n * mul) >> 32 >> shift, with mul =
+// ceil(2^(31+l) / d), 2^(l-1) < d <= 2^l and shift = l - 1 (mul exceeds the
+// quotient by less than 1, so the product by less than 2^31 / 2^(31+l) <= 1 / d).
+struct Div {
+    uint32_t d, mul;
+    int shift;
+    __device__ __forceinline__ uint32_t operator()(uint32_t n) const { return __umulhi(n, mul) >> shift; }
+};
+
+inline Div make_div(uint32_t d) {
+    int l = 1;
+    while ((uint64_t{1} << l) < d) ++l;
+    return {d, static_cast<uint32_t>(((uint64_t{1} << (31 + l)) + d - 1) / d), l - 1};
+}
+
+// v of lane l ^ M as a DPP source (no LDS): M = 1 and 2 within 4 lanes, M = 8 the
+// rotation by 8 of 16.  For M = 4 the rotation by 4, which reads lane l ^ 4 or
+// l ^ 12: for values that lanes 8 apart share.
+template <int M>
+__device__ __forceinline__ float dpp_xor(float v) {
+    constexpr int ctrl = M == 1 ? 0xB1 : M == 2 ? 0x4E : M == 4 ? 0x124 : 0x128;
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "DPP pattern");
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, 0xF, true));
+}
+
+// v plus the v of lane l ^ M, in a butterfly over LPR lanes from LPR / 2 down (so
+// that from M = 4 down, lanes 2 M apart hold the same v).
+template <int LPR, int M>
+__device__ __forceinline__ float butterfly(float v) {
+    if constexpr (M == 16 || (M == 4 && LPR == 8)) return v + __shfl_xor(v, M, 64);
+    else return v + dpp_xor<M>(v);
+}
+
 // One wave handles NIT sets of 64 / LPR rows; every load of the wave is
 // issued before the first row is reduced, so a wave keeps NIT x 1 KiB of rows
-// (plus their table entries) in flight.  Branches around memory operations
-// make the compiler drain all loads at the join, so the bulk launch covers
-// whole workgroups (GUARD = false: no row test) and a second, guarded launch
-// takes the remaining rows; RSTD (the per-row rstd output) is for tests;
-// ROPE: 0 no rotation (rot = 0), 2 full rotation (rot = D), 1 partial; with
-// a rotation every lane loads table words (lanes outside a partial rotation
-// load pair 0 and ignore it) so no branch surrounds the loads;
-// RN selects the correctly rounded rsqrt (else the hardware one, as eager).
+// in flight.  Branches around memory operations make the compiler drain all
+// loads at the join, so a row past the end loads row 0 instead (unused) and
+// only the stores test the row.  RSTD (the per-row rstd output) is for tests;
+// ROPE: 0 no rotation (rot = 0), 2 full rotation (rot = D), 1 partial; RN
+// selects the correctly rounded rsqrt (else the hardware one, as eager).
 //
-// VALU economy (about 20 instructions per element, so the shader clock
-// shows in the kernel's time):
-// each lane loads exactly the 8 table words it uses (lower lanes word 0 =
-// R00 | R01 << 16 of its 8 pairs, upper lanes word 1 = R10 | R11 << 16), so no
-// table words are exchanged or selected; the weights are staged once per
-// workgroup in LDS as fp32, q's then k's; the cross-lane sums and the partner
-// values go over the LDS crossbar.
-template <int LPR, int NIT, bool GUARD, bool RSTD, int ROPE, bool RN>
+// The weights (q's then k's) and the table rows of the workgroup's tokens are
+// staged in LDS as fp32, the table as four planes of rot/2 coefficients per
+// token (R00, R01, R10, R11), so a lane takes its eight pairs' two coefficients
+// as four 16-byte reads, ready to multiply.  Loaded per row instead, each
+// lane's own eight table words, a wave held 32 registers of them and fetched
+// each table line eight times (and one way or the other waited for them before
+// the next set's rows went out).  The reduction and, at a full rotation of 16
+// lanes, the partner's value are DPP sources; over the LDS crossbar their
+// latency showed (19200 tokens of 56 x 128 196 against 182 us).  With the one
+// launch for every row count (the rest of the rows was a second, guarded one),
+// tokens of 56 x 128, before -> after: 37 10.1 -> 4.0 us, 512 9.6 -> 7.2, 2401 33
+// -> 25.9, 19200 187 -> 182 (6.1 TB/s: memory).
+template <int LPR, int NIT, bool RSTD, int ROPE, bool RN>
 __global__ __launch_bounds__(256) void rms_rope_kernel(uint16_t* __restrict__ q, uint16_t* __restrict__ k,
                                                        const uint16_t* __restrict__ tab,
                                                        const uint16_t* __restrict__ qw,
-                                                       const uint16_t* __restrict__ kw, int S, int H, int64_t ldq,
-                                                       int64_t ldk, int rot, float eps, int mode,
-                                                       float* __restrict__ rstd_out, int64_t row_base) {
+                                                       const uint16_t* __restrict__ kw, int S, int H, Div per_tok,
+                                                       int64_t ldq, int64_t ldk, int rot, float eps,
+                                                       float* __restrict__ rstd_out) {
 #pragma clang fp contract(off)
     constexpr int D = LPR * 8;
     constexpr int RPW = 64 / LPR;
+    constexpr int RPB = 4 * RPW * NIT;
     static_assert(D <= 256, "one weight element per thread of the workgroup");
-    __shared__ __attribute__((aligned(16))) float wsh[2 * D];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    float* const wsh = smem;          // [2][D]
+    float* const tsh = smem + 2 * D;  // [tokens][4][rot / 2]
     const int lane = threadIdx.x & 63;
     const int sub = lane % LPR;
-    const int64_t rows = static_cast<int64_t>(S) * 2 * H;
-    const int64_t row0 =
-        row_base + (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * (RPW * NIT) + lane / LPR;
+    const uint32_t rows = static_cast<uint32_t>(S) * per_tok.d;  // < 2^31 (checked by the caller)
+    const uint32_t block0 = blockIdx.x * static_cast<uint32_t>(RPB);
+    const uint32_t row0 = block0 + (threadIdx.x >> 6) * (RPW * NIT) + lane / LPR;
+    const uint32_t tok0 = per_tok(block0);  // uniform: the workgroup's first token
     // rotation: lanes [0, rot/16) of a row hold the first halves, [rot/16,
     // rot/8) the second halves, the partner lane rot/16 away
-    const int hl = rot / 16;
+    const int hl = rot / 16, half = rot / 2;
     const bool lower = sub < hl;
     const bool rotated = ROPE == 2 || sub < 2 * hl;
     const int src = rotated ? (lower ? lane + hl : lane - hl) : lane;
     const int pair0 = rotated ? (lower ? sub : sub - hl) * 8 : 0;
-    const int word = (rotated && !lower) ? 1 : 0;
-    // v_perm selectors (bytes 4-7 = first operand, 0x0c = zero): the low half
-    // of a word as an fp32 is bytes {5, 4} on top, the high half bytes {7, 6}
-    const uint32_t sel_lo = 0x05040C0Cu, sel_hi = 0x07060C0Cu;
-    const uint32_t sel_own = lower ? sel_lo : sel_hi, sel_par = lower ? sel_hi : sel_lo;
 
-    // the weights first (loads complete in order): thread t stages element
-    // t % D of both; threads past D write the same values again
+    // the weights and the table first (loads complete in order): thread t takes
+    // element t % D of both weights (threads past D write the same values again)
     const int wt = static_cast<int>(threadIdx.x) % D;
     const uint16_t wq1 = qw[wt], wk1 = kw[wt];
+    const int last = static_cast<int>(per_tok(min(block0 + RPB, rows) - 1) - tok0);  // of its tokens
+    const uint2* const pt = reinterpret_cast<const uint2*>(tab) + static_cast<int64_t>(tok0) * half;
+    const int pairs = ROPE > 0 ? (last + 1) * half : 0;
+    uint2 t0 = make_uint2(0u, 0u);
+    if (ROPE > 0 && static_cast<int>(threadIdx.x) < pairs) t0 = pt[threadIdx.x];
+    __builtin_amdgcn_sched_barrier(0);  // moved behind the rows' loads, their wait would drain them all
 
-    // rows < 2^31 (checked by the caller), so 32-bit arithmetic; one division
-    // for the wave's first set, then steps of RPW rows
-    const uint32_t rows_per_tok = 2u * static_cast<uint32_t>(H);
-    uint32_t tok = static_cast<uint32_t>(row0) / rows_per_tok;
-    uint32_t jr = static_cast<uint32_t>(row0) - tok * rows_per_tok;
-    int64_t row[NIT];
     bool in[NIT], isk[NIT];
+    uint32_t rel[NIT];
     uint16_t* px[NIT];
     v4u_t xv[NIT];
-    uint32_t tw[NIT][8];
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-        if (it > 0) {
-            jr += RPW;
-            while (jr >= rows_per_tok) {
-                jr -= rows_per_tok;
-                ++tok;
-            }
-        }
-        row[it] = row0 + static_cast<int64_t>(it) * RPW;
-        in[it] = !GUARD || row[it] < rows;
-        const uint32_t t32 = in[it] ? tok : 0u;
-        const int j = static_cast<int>(jr);
+        const uint32_t row = row0 + it * RPW;
+        in[it] = row < rows;
+        const uint32_t r = in[it] ? row : block0;
+        const uint32_t tok = per_tok(r);
+        const int j = static_cast<int>(r - tok * per_tok.d);
+        rel[it] = tok - tok0;
         isk[it] = j >= H;
-        px[it] = (isk[it] ? k + static_cast<int64_t>(t32) * ldk : q + static_cast<int64_t>(t32) * ldq) +
+        px[it] = (isk[it] ? k + static_cast<int64_t>(tok) * ldk : q + static_cast<int64_t>(tok) * ldq) +
                  static_cast<int64_t>(isk[it] ? j - H : j) * D + sub * 8;
-        xv[it] = v4u_t{0u, 0u, 0u, 0u};
-        if (!GUARD || in[it]) xv[it] = __builtin_nontemporal_load(reinterpret_cast<const v4u_t*>(px[it]));
-        if constexpr (ROPE > 0) {
-            // rows past the end (GUARD) have token 0, whose table row exists;
-            // pair m's words are elements 4m .. 4m+3 of the table row
-            const uint32_t* pt = reinterpret_cast<const uint32_t*>(tab + (static_cast<int64_t>(t32) * (rot / 2) + pair0) * 4) + word;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) tw[it][i] = pt[2 * i];
-        }
+        xv[it] = __builtin_nontemporal_load(reinterpret_cast<const v4u_t*>(px[it]));
     }
     __builtin_amdgcn_sched_barrier(0);  // every load above is issued before any row is reduced
     wsh[wt] = bf16_f32(wq1);
     wsh[D + wt] = bf16_f32(wk1);
+    if constexpr (ROPE > 0) {
+        auto stage = [&](int p, uint2 w) {
+            float* const d = tsh + (p / half) * 4 * half + p % half;
+            d[0] = bf16_lo(w.x);
+            d[half] = bf16_hi(w.x);
+            d[2 * half] = bf16_lo(w.y);
+            d[3 * half] = bf16_hi(w.y);
+        };
+        if (static_cast<int>(threadIdx.x) < pairs) stage(threadIdx.x, t0);
+        for (int p = threadIdx.x + 256; p < pairs; p += 256) stage(p, pt[p]);  // few heads: many tokens
+    }
     wait_lgkm0();  // the writes are done
     wg_barrier();
 
@@ -144,16 +176,23 @@ __global__ __launch_bounds__(256) void rms_rope_kernel(uint16_t* __restrict__ q,
             pe = pe + x[i] * x[i];
             po = po + x[4 + i] * x[4 + i];
         }
-#pragma unroll
-        for (int d = LPR / 2; d >= 1; d /= 2) {
-            pe = pe + __shfl_xor(pe, d, 64);
-            po = po + __shfl_xor(po, d, 64);
-        }
+        auto both = [&](auto m_c) {
+            constexpr int M = decltype(m_c)::value;
+            if constexpr (M < LPR) {
+                pe = butterfly<LPR, M>(pe);
+                po = butterfly<LPR, M>(po);
+            }
+        };
+        both(std::integral_constant<int, 16>{});
+        both(std::integral_constant<int, 8>{});
+        both(std::integral_constant<int, 4>{});
+        both(std::integral_constant<int, 2>{});
+        both(std::integral_constant<int, 1>{});
         // D is a power of two: the product by 1/D is the IEEE quotient
         const float var = (pe + po) * (1.0f / static_cast<float>(D)) + eps;
         const float rstd = RN ? rsqrt_rn(var) : rsqrtf(var);
         if constexpr (RSTD) {
-            if (in[it] && sub == 0) rstd_out[row[it]] = rstd;
+            if (in[it] && sub == 0) rstd_out[row0 + it * RPW] = rstd;
         }
 
         const float* wr = wsh + (isk[it] ? D : 0) + sub * 8;
@@ -165,27 +204,34 @@ __global__ __launch_bounds__(256) void rms_rope_kernel(uint16_t* __restrict__ q,
 #pragma unroll
         for (int i = 0; i < 4; ++i) rb2(y[2 * i], y[2 * i + 1]);
         if constexpr (ROPE > 0) {
+            // lower lane: out = R00 y + R01 p; upper lane: R10 p + R11 y, the
+            // same sum in the other order
+            const float* tr = tsh + rel[it] * 4 * half + pair0;
+            const float* const po_ = tr + (lower ? 0 : 3 * half);
+            const float* const pp_ = tr + (lower ? half : 2 * half);
+            const float4 o0 = *reinterpret_cast<const float4*>(po_), o1 = *reinterpret_cast<const float4*>(po_ + 4);
+            const float4 q0 = *reinterpret_cast<const float4*>(pp_), q1 = *reinterpret_cast<const float4*>(pp_ + 4);
+            const float co[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
+            const float cp[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
             float p[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) p[i] = __shfl(y[i], src, 64);
-            if (rotated) {
+            for (int i = 0; i < 8; ++i) {
+                if constexpr (ROPE == 2 && LPR == 16) p[i] = dpp_xor<8>(y[i]);  // rot / 16 lanes apart
+                else p[i] = __shfl(y[i], src, 64);
+            }
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    // lower lane: out = R00 y + R01 p; upper lane: R10 p + R11 y,
-                    // the same sum in the other order; c_own / c_par pick the
-                    // halves of the lane's word by a per-lane selector
-                    const float c_own = __uint_as_float(__builtin_amdgcn_perm(tw[it][i], 0u, sel_own));
-                    const float c_par = __uint_as_float(__builtin_amdgcn_perm(tw[it][i], 0u, sel_par));
-                    const float u = c_own * y[i];
-                    const float v = c_par * p[i];
-                    y[i] = u + v;
-                }
+            for (int i = 0; i < 8; ++i) {
+                const float u = co[i] * y[i];
+                const float v = cp[i] * p[i];
+                y[i] = rotated ? u + v : y[i];
             }
         }
         v4u_t ov;
 #pragma unroll
         for (int i = 0; i < 4; ++i) ov[i] = bf16x2_bits(y[2 * i], y[2 * i + 1]);
-        if (!GUARD || in[it]) __builtin_nontemporal_store(ov, reinterpret_cast<v4u_t*>(px[it]));
+        // opaque: else the compiler moves the rotation into the store's branch
+        asm volatile("" : "+v"(ov));
+        if (in[it]) __builtin_nontemporal_store(ov, reinterpret_cast<v4u_t*>(px[it]));
     }
 }
 
@@ -230,24 +276,34 @@ extern "C" int h3mi_rms_rope_split_half_bf16(uint16_t* q, uint16_t* k, const uin
         const size_t rb_ = static_cast<size_t>(S * 2 * H) * 4;
         if (overlap(rstd_out, rb_, q, qb) || overlap(rstd_out, rb_, k, kb)) return fail(H3MI_EALIAS, "rms_rope: rstd_out overlaps q/k");
     }
-    constexpr int NIT = 4;
     const int lpr = static_cast<int>(D / 8);
     const int64_t rows = S * 2 * H;
-    const int64_t rows_per_block = 4 * (64 / lpr) * NIT;
-    const int64_t full = rows / rows_per_block;  // workgroups whose rows all exist
-    const int64_t tail = rows - full * rows_per_block;
-    auto launch = [&](auto kern, int64_t blocks, int64_t base) {
-        if (blocks <= 0) return;
-        hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream), q, k, tab, qw, kw,
-                           static_cast<int>(S), static_cast<int>(H), ldq, ldk, static_cast<int>(rot), eps, rsqrt_mode_,
-                           rstd_out, base);
+    const Div per_tok = make_div(static_cast<uint32_t>(2 * H));
+    // Four sets of rows per wave, or two where four would leave a CU fewer than
+    // four workgroups (512 tokens of 56 x 128 7.9 against 8.8 us, 37 4.3 against
+    // 4.7; 1024 14.2 against 13.5; before the DPP sources).
+    const bool few = rows / (16 * (64 / lpr)) < 4 * static_cast<int64_t>(cu_count());
+    auto run4 = [&](auto lpr_c, auto rstd_c, auto rope_c, auto rn_c, auto nit_c) {
+        constexpr int L = decltype(lpr_c)::value, NIT = decltype(nit_c)::value, P = decltype(rope_c)::value;
+        constexpr bool R = decltype(rstd_c)::value, N = decltype(rn_c)::value;
+        constexpr int64_t rows_per_block = 4 * (64 / L) * NIT;
+        const unsigned blocks = static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block);
+        // the weights, and the table rows of as many tokens as a workgroup's rows can touch
+        const int64_t toks = (rows_per_block - 2) / (2 * H) + 2;
+        size_t lds = static_cast<size_t>(2 * D + (rot ? toks * 2 * rot : 0)) * sizeof(float);
+        // Rows that come from memory stream faster with five workgroups per CU
+        // than with the seven that the registers allow, so the LDS of a long
+        // launch is padded: 19200 tokens of 56 x 128 182 against 187 us, 40 x 128
+        // 133.5 against 141, 2401 of 56 25.9 against 26.4; 1024 (29 MB) 13.1
+        // against 12.3.
+        if (rows * D * 2 >= int64_t{48} << 20 && lds < 32768) lds = 32768;
+        hipLaunchKernelGGL((rms_rope_kernel<L, NIT, R, P, N>), dim3(blocks), dim3(256), lds, as_stream(stream), q, k, tab,
+                           qw, kw, static_cast<int>(S), static_cast<int>(H), per_tok, ldq, ldk, static_cast<int>(rot), eps,
+                           rstd_out);
     };
     auto run3 = [&](auto lpr_c, auto rstd_c, auto rope_c, auto rn_c) {
-        constexpr int L = decltype(lpr_c)::value;
-        constexpr bool R = decltype(rstd_c)::value, N = decltype(rn_c)::value;
-        constexpr int P = decltype(rope_c)::value;
-        launch(rms_rope_kernel<L, NIT, false, R, P, N>, full, 0);
-        launch(rms_rope_kernel<L, NIT, true, R, P, N>, tail ? 1 : 0, full * rows_per_block);
+        if (few) run4(lpr_c, rstd_c, rope_c, rn_c, std::integral_constant<int, 2>{});
+        else run4(lpr_c, rstd_c, rope_c, rn_c, std::integral_constant<int, 4>{});
     };
     using T = std::true_type;
     using F = std::false_type;

@@ -161,3 +161,11 @@ def test_h3_size_matches_eager():
     k = buf[:, H * D:2 * H * D].view(1, S, H, D)
     h.rms_rope_split_half_(q, k, tab[None], qw, kw, epsilon=eps)
     assert torch.equal(q[0], refq) and torch.equal(k[0], refk) and torch.equal(buf[:, 2 * H * D:], v0)
+
+
+@pytest.mark.parametrize("S,H,D,rot", [(1501, 47, 128, 96), (1801, 12, 256, 256), (3001, 24, 64, 32), (65, 1, 128, 128),
+                                       (513, 56, 128, 128)])
+def test_rest_rows_and_many_tokens_match_eager_and_oracle(S, H, D, rot):
+    """Row counts that leave a part of a workgroup, in launches of four and of
+    two row sets per wave, and workgroups whose rows span many tokens."""
+    test_matches_eager_and_oracle(S, H, D, rot)
