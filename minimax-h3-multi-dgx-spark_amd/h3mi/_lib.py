@@ -77,6 +77,12 @@ def _load():
 
 lib = _load()
 
+import torch  # noqa: E402,F401  (its libraries, which _fast links)
+
+from . import _fast  # noqa: E402  (the common calls in native code; like libh3mi.so, built by the Makefile)
+
+_fast.set_error(H3miError)
+
 
 def check(status):
     if status != OK:

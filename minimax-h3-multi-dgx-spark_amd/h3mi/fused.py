@@ -16,7 +16,7 @@ import ctypes
 
 import torch
 
-from ._lib import ORDER_DEFAULT, RSQRT_HW, check, lib, ptr, same_gpu, stream_of
+from ._lib import ORDER_DEFAULT, RSQRT_HW, _fast, check, lib, ptr, same_gpu, stream_of
 
 ORDER_NAMES = {"default": 0, "ref": 1, "w64": 2}
 
@@ -95,7 +95,15 @@ def gate_norm_mod_ex(x, o, g, w, eps, ridx, s1, sh, order=ORDER_DEFAULT, rsqrt_m
     return (h, var, rstd) if stats else h
 
 
+# The four norms below and gate_ first offer the call to native code, which takes
+# it in the plain form (csrc/fastcall.cpp) or returns None; the checks here then
+# decide every other form.
+
+
 def norm_mod(x, w, eps, ridx, s1, sh):
+    h = _fast.norm_mod(x, w, eps, ridx, s1, sh, False)
+    if h is not None:
+        return h
     s, n = _rows(x)
     _weight(w, n)
     _ridx(ridx, s)
@@ -110,6 +118,9 @@ def norm_mod(x, w, eps, ridx, s1, sh):
 
 
 def gate_norm_mod_(x, o, g, w, eps, ridx, s1, sh):
+    h = _fast.gate_norm_mod_(x, o, g, w, eps, ridx, s1, sh, False)
+    if h is not None:
+        return h
     s, n = _rows(x)
     if o.shape != x.shape or o.dtype != torch.bfloat16 or not o.is_contiguous():
         raise ValueError("o must be contiguous bfloat16 like x")
@@ -126,6 +137,9 @@ def gate_norm_mod_(x, o, g, w, eps, ridx, s1, sh):
 
 
 def gate_(x, o, g, ridx):
+    y = _fast.gate_(x, o, g, ridx)
+    if y is not None:
+        return y
     s, n = _rows(x)
     if o.shape != x.shape or o.dtype != torch.bfloat16 or not o.is_contiguous():
         raise ValueError("o must be contiguous bfloat16 like x")
@@ -144,6 +158,10 @@ def norm_mod_q(x, w, eps, ridx, s1, sh, want_h=False):
     """norm_mod with the per-token quantizer of h fused in.  Returns (q, qs),
     or (h, q, qs) with want_h.  Rows the fused kernel does not take (N % 8 != 0
     or N > 8192) run norm_mod then quantize_rowwise."""
+    if not want_h:
+        r = _fast.norm_mod(x, w, eps, ridx, s1, sh, True)
+        if r is not None:
+            return r
     s, n = _rows(x)
     _weight(w, n)
     _ridx(ridx, s)
@@ -167,6 +185,10 @@ def norm_mod_q(x, w, eps, ridx, s1, sh, want_h=False):
 def gate_norm_mod_q_(x, o, g, w, eps, ridx, s1, sh, want_h=False):
     """gate_norm_mod_ (x updated in place) with the per-token quantizer of h
     fused in.  Returns (q, qs), or (h, q, qs) with want_h."""
+    if not want_h:
+        r = _fast.gate_norm_mod_(x, o, g, w, eps, ridx, s1, sh, True)
+        if r is not None:
+            return r
     s, n = _rows(x)
     if o.shape != x.shape or o.dtype != torch.bfloat16 or not o.is_contiguous():
         raise ValueError("o must be contiguous bfloat16 like x")

@@ -31,7 +31,7 @@ import re
 
 import torch
 
-from ._lib import H3miError, check, lib, ptr, same_gpu, stream_of
+from ._lib import H3miError, _fast, check, lib, ptr, same_gpu, stream_of
 
 log = logging.getLogger("h3mi")
 
@@ -39,7 +39,8 @@ log = logging.getLogger("h3mi")
 class _KernelInfo:
     """Stand-in for the autotuned kernel object: best_config names the tile
     configuration the last call used.  It is looked up when read, not on every
-    call (a ctypes round trip per GEMM launch otherwise)."""
+    call (a ctypes round trip per GEMM launch otherwise).  The native calls keep
+    their last shape themselves."""
 
     def __init__(self):
         self._shape = None  # (M, N, K) of the last call that took the heuristic
@@ -47,9 +48,13 @@ class _KernelInfo:
 
     def _record(self, shape=None, name=None):
         self._shape, self._name = shape, name
+        _fast.last_shape(False)
 
     @property
     def best_config(self):
+        fast = _fast.last_shape(True)
+        if fast is not None:
+            return config_for(*fast)
         if self._name is not None:
             return self._name
         return config_for(*self._shape) if self._shape is not None else None
@@ -162,6 +167,10 @@ def int8_mm_scaled(xq, w, xs, ws, out=None, bias=None):
 
     out[m,n] = bf16((f32(sum_k xq[m,k]*w[n,k]) * xs[m]) * ws[n])
     (+ bias[n] in fp32 before the rounding when bias, bf16 [N], is given)."""
+    if out is None:
+        y = _fast.int8_mm_scaled(xq, w, xs, ws, bias)
+        if y is not None:
+            return y
     M, N, K = _check_operands(xq, w)
     if xs.dtype != torch.float32 or xs.numel() != M or not xs.is_contiguous():
         raise ValueError("xs must be contiguous float32 with M elements")

@@ -7,11 +7,15 @@ for an all-zero row.
 """
 import torch
 
-from ._lib import check, lib, ptr, same_gpu, stream_of
+from ._lib import _fast, check, lib, ptr, same_gpu, stream_of
 
 
 def quantize_rowwise(x, xq=None, xs=None):
     """x bf16 [M,K] (row stride may exceed K) -> (xq int8 [M,K], xs fp32 [M,1])."""
+    if xq is None and xs is None:
+        r = _fast.quantize(x, -1)
+        if r is not None:
+            return r
     if x.dim() != 2 or x.dtype != torch.bfloat16 or not x.is_cuda:
         raise ValueError("x must be a 2-D bfloat16 GPU tensor")
     if x.stride(1) != 1:
@@ -44,6 +48,10 @@ def quantize_rowwise_convrot(x, act=None, group_size=256, xq=None, xs=None):
     xq = clamp(rne(y/xs), -127, 127).  K % 256 == 0, K <= 32768."""
     if act not in _ACTS:
         raise ValueError(f"unsupported input activation {act!r}")
+    if xq is None and xs is None and group_size == 256:
+        r = _fast.quantize(x, _ACTS[act])
+        if r is not None:
+            return r
     if x.dim() != 2 or x.dtype != torch.bfloat16 or not x.is_cuda:
         raise ValueError("x must be a 2-D bfloat16 GPU tensor")
     if x.stride(1) != 1:

@@ -11,7 +11,7 @@ table entry i, in fp32, rounded to bf16.
 """
 import torch
 
-from ._lib import RSQRT_HW, RSQRT_RN, check, lib, ptr, same_gpu, stream_of
+from ._lib import RSQRT_HW, RSQRT_RN, _fast, check, lib, ptr, same_gpu, stream_of
 
 _MODES = {"hw": RSQRT_HW, "rn": RSQRT_RN}
 
@@ -34,6 +34,10 @@ def _rows(t, name):
 def rms_rope_split_half_(q, k, rope_freqs, qw, kw, epsilon=1e-6, rot_dim=None, rsqrt="hw", rstd_out=None):
     """In place on q and k; returns (q, k).  rope_freqs: [..., s, rot/2, 2, 2]
     bf16 (leading singleton dimensions allowed), or None with rot_dim 0."""
+    if rsqrt == "hw" and rstd_out is None:
+        r = _fast.rms_rope_(q, k, rope_freqs, qw, kw, epsilon, rot_dim)
+        if r is not None:
+            return r
     q3, S, H, D, ldq = _rows(q, "q")
     k3, Sk, Hk, Dk, ldk = _rows(k, "k")
     if (Sk, Hk, Dk) != (S, H, D):
