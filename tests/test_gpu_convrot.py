@@ -176,3 +176,18 @@ def test_convrot_empty_and_rejects():
         h.quantize_rowwise_convrot(torch.zeros(4, 1000, dtype=torch.bfloat16, device="cuda"))
     with pytest.raises(ValueError):
         h.quantize_rowwise_convrot(torch.zeros(4, 1024, dtype=torch.bfloat16, device="cuda"), act="gelu")
+
+
+@pytest.mark.parametrize("act", [None, "swiglu"])
+@pytest.mark.parametrize("K", [256, 2048, 2560, 3072, 5376, 7168, 14336, 24832])
+def test_many_rows_equal_few(K, act):
+    """The wave and pass shapes of long calls give the bytes of those of short
+    ones (which the other tests hold against the oracle)."""
+    import h3mi
+    M = 1601
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(M, K * (2 if act else 1), generator=g, device="cuda").to(torch.bfloat16)
+    q, s = h3mi.quantize_rowwise_convrot(x, act)
+    parts = [h3mi.quantize_rowwise_convrot(x[i:i + 160], act) for i in range(0, M, 160)]
+    assert torch.equal(q, torch.cat([p[0] for p in parts]))
+    assert torch.equal(s.view(torch.int32), torch.cat([p[1] for p in parts]).view(torch.int32))
