@@ -353,7 +353,9 @@ __device__ __forceinline__ void store_tile_lds_impl(const v16i (&acc)[T::FN][T::
                 uint16_t* o = out + static_cast<int64_t>(m) * ldo + n;
                 if (m < M && n < N) {
                     if (n + 8 <= N) {
-                        __builtin_nontemporal_store(v, reinterpret_cast<v4u*>(o));
+                        // cached: see store_tile_lds (A1 tiles get whole-line rows)
+                        if constexpr (T::A1) __builtin_nontemporal_store(v, reinterpret_cast<v4u*>(o));
+                        else *reinterpret_cast<v4u*>(o) = v;
                     } else {  // N % 4 == 0: the row ends half-way through this chunk
                         __builtin_nontemporal_store(v2u{v[0], v[1]}, reinterpret_cast<v2u*>(o));
                     }
@@ -370,7 +372,14 @@ __device__ __forceinline__ void store_tile_lds(const v16i (&acc)[T::FN][T::FM], 
     // Uniform branches around the whole epilogue, none inside it: bias or
     // not, and whether the workgroup tile lies wholly inside the output (and
     // eight output rows span under 2^31 bytes, so lane offsets fit 32 bits).
-    const bool full = m0 + T::BM <= M && n0 + T::BN <= N && ldo < (int64_t{1} << 27);
+    // Rows that do not start on a 128-byte line (N = 9000) take the bounds-checked
+    // variant too, whose stores are cached: a slab's segment of a row ends inside
+    // two lines whose other parts the neighbouring slabs write, and non-temporal
+    // stores sent each part to memory by itself; the L2 joins them (10000 x 9000
+    // x 384 69 against 108 us, x 1536 147 against 167).  A copy of the unchecked
+    // variant with cached stores cost the other shapes 1% by its size alone.
+    const bool lines = T::A1 || ((ldo & 63) == 0 && (reinterpret_cast<uintptr_t>(out) & 127) == 0);
+    const bool full = lines && m0 + T::BM <= M && n0 + T::BN <= N && ldo < (int64_t{1} << 27);
     if (has_bias) {
         if (full) store_tile_lds_impl<T, true, true, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
         else store_tile_lds_impl<T, true, false, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
@@ -1026,11 +1035,10 @@ int wave_split_or(int other, int64_t M, int64_t N, int64_t K, int64_t cus) {
 
 // Big grids (at least two 256x256 tiles per CU) run one resident workgroup
 // per CU over the tiles.  Of the 256x256, 256x384, 320x256 and 256x320
-// tilings, the one whose busiest workgroup has the least work runs: its tile
-// count rounded up to whole rounds over the CUs, times the tile area, with the
-// 256x384 and 256x320 tiles' measured 3% and 2.4% higher rates per area.  Of the
-// smaller grids, one of the 128x128, 128x192 or larger tiles is weighed by the
-// same measure and then against the wave-split tilings by predicted time.
+// tilings, the one whose busiest workgroup has the least work runs (below).  Of
+// the smaller grids, one of the 128x128, 128x192 or larger tiles is picked by
+// whole rounds over the CUs times tile area and then weighed against the
+// wave-split tilings by predicted time.
 int pick_config(int64_t M, int64_t N, int64_t K) {
     {
         // a forced configuration that cannot take this K (split-K tilings
@@ -1056,6 +1064,10 @@ int pick_config(int64_t M, int64_t N, int64_t K) {
     // work per CU: N = 15360 and 5120); with a ragged last column (N = 5376)
     // they measured 3-4% slower than 320x256, so they are offered only then.
     const bool n320 = N % 320 == 0;
+    // 256x384 tiles are offered when output rows start on 128-byte lines: their
+    // epilogue has no room for the cached stores that other rows want
+    // (32768 x 9000 x 5120 1300 against 1208 us, x 768 515 against 306).
+    const bool lines = N % 64 == 0;
     const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
     if (t256 < 2 * cus) {
         // Fewer than two 256x256 tiles per CU: 128x128 tiles (two workgroups
@@ -1082,7 +1094,7 @@ int pick_config(int64_t M, int64_t N, int64_t K) {
         // 768 x 28672 x 5376 110 against 138 us, 1536 x 15360 x 5120 98 against
         // 116, 4096 x 5376 x 14336 260 against 327; with a short K its epilogue
         // weighs more (2400 x 9000 x 1536: 58.6 against 53.3).
-        const double c384 = K >= 3072 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
+        const double c384 = lines && K >= 3072 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
         const double ck2 = K % 256 == 0 ? rounds(128, 192) * 128.0 * 192.0 / 0.88 : 1e300;
         int c = c256 < c128 ? big : small;
         if (ck2 < c256 && ck2 < c128) c = split;
@@ -1095,10 +1107,16 @@ int pick_config(int64_t M, int64_t N, int64_t K) {
         if (c == small && t128 <= cus && K % 256 == 0 && K >= 4096) c = small_k2;
         return wave_split_or(c, M, N, K, cus);
     }
-    const double w256 = rounds(256, 256) * 256.0 * 256.0;
-    const double w384 = rounds(256, 384) * 256.0 * 384.0 / 1.03;
-    const double w320 = rounds(320, 256) * 320.0 * 256.0;
-    const double w320n = n320 ? rounds(256, 320) * 256.0 * 320.0 / 1.024 : 1e300;
+    // Work of the busiest CU: rounds times tile area times K plus what a tile
+    // costs beside its K loop (as that many K), over the tiling's rate.  Fitted
+    // to 110 shapes of K 384 to 5120 (M 3500 to 32768, N 3072 to 21504): the
+    // picked tiling is 0.9% slower than the fastest on average, 6.5% for tile
+    // areas alone, which sent short K to 256x384 tiles (10000 x 13824 x 384 110
+    // against 88 us, 32768 x 13824 x 768 439 against 383).
+    const double w256 = rounds(256, 256) * 256.0 * 256.0 * (K + 554);
+    const double w384 = lines ? rounds(256, 384) * 256.0 * 384.0 * (K + 820) / 1.07 : 1e300;
+    const double w320 = rounds(320, 256) * 320.0 * 256.0 * (K + 541);
+    const double w320n = n320 ? rounds(256, 320) * 256.0 * 320.0 * (K + 640) / 1.024 : 1e300;
     if (w320n < w256 && w320n < w384 && w320n < w320) return flat;
     if (w384 < w256 && w384 <= w320) {
         // Operands past ~240 MiB (the 256 MB infinity cache, less what else
