@@ -18,6 +18,7 @@
 #include <utility>
 
 #include "common.h"
+#include "norm_route.h"
 
 namespace h3mi {
 namespace {
@@ -1276,7 +1277,7 @@ __global__ __launch_bounds__(256) void gate_norm_split_kernel(
 // ------------------------------------------------------------------ one row per workgroup, not persistent
 
 // For calls whose tensors the caches still hold or whose rows are few per CU,
-// and for tables of several rows (rows_suit below).  There the row streams'
+// and for tables of several rows (norm_rows_suit).  There the row streams'
 // set-up -- counting the table rows, copying them to LDS as fp32, a barrier
 // each -- and the one or two rows that a wave has in flight are most of the
 // call, and a row whose table row is not the staged one reads its tables late.
@@ -1401,30 +1402,6 @@ __global__ __launch_bounds__(256) void gate_row_kernel(uint16_t* __restrict__ x,
     for (int it = 0; it < IT; ++it) store_row16(xr, it * 2048 + 8 * t, gate8(X[it], O[it], G[it]));
 }
 
-// Whether a call of S rows runs the one-row-per-workgroup kernels (gate_ has its
-// own line).  With one table row the streams win once the tensors come from
-// memory (with inputs rotated past the caches the two meet at about 16 Mi
-// elements, 24 Mi with the quantizer, whose streams have less of a row in
-// flight), and, in rows narrower than a workgroup, past about 20 rows per CU
-// (at N = 512 9600 rows: norm_mod 12.5 against 14.0 us, norm_mod_q 16.8 against
-// 14.6); gate_norm_mod_'s own stream, a workgroup per row and CU, is behind at
-// any S for N = 1024 to 2048 (38400 x 1024: 106.7 against 67.9).  With several
-// table rows a stream reads most rows' tables from L2 after their x, and the
-// lines move: 38400 x 5376 over five, gate_norm_mod_ 470 against 323 us,
-// gate_norm_mod_q_ 380 against 325, norm_mod 209 against 201, but norm_mod_q 170
-// against 188; over two, gate_norm_mod_ 361 against 325, gate_norm_mod_q_ 175
-// against 172 at 19200 rows and 303 against 319 at 38400, norm_mod 30.4 against
-// 28.7 at 4800 and 52 against 57 at 9600.
-bool rows_suit(bool gate, bool quant, int64_t S, int64_t N, int64_t R) {
-    const int64_t mi = S * N >> 20;
-    if (R > 1) {
-        if (gate) return !quant || R > 3 || mi < 100;
-        return quant ? mi < 32 : R > 3 || mi < 24;
-    }
-    if (gate && !quant && N >= 1024 && N <= 2048) return true;
-    return S <= 5120 && mi < (quant ? 24 : 16);
-}
-
 template <bool GATE, int QUANT>
 int launch_rows(uint16_t* x, const uint16_t* o, const uint16_t* g, const uint16_t* w, const int32_t* ridx,
                 const uint16_t* s1, const uint16_t* sh, uint16_t* h, int64_t S, int N, int R, float eps, int rsq,
@@ -1448,7 +1425,7 @@ int launch_order(uint16_t* x, const uint16_t* o, const uint16_t* g, const uint16
     // Persistent row stream for N <= 8192 in the product order; the reference
     // order (a parity mode) keeps the kernels below.
     const int ch = (NUMX == 256 && WARP == 64) ? stream_ch(N) : 0;
-    if (ch > 0 && rows_suit(GATE, false, S, N, R))
+    if (ch > 0 && norm_rows_suit(GATE, false, S, N, R))
         return launch_rows<GATE, 0>(x, o, g, w, ridx, s1, sh, h, S, N, R, eps, rsq, var, rstd, nullptr, nullptr, st,
                                     GATE ? "gate_norm_mod" : "norm_mod");
     if (GATE && ch > 0 && N >= 1024 && (N % 1024 == 0 || N % 1024 == 256)) {
@@ -1576,7 +1553,7 @@ int norm_quant_entry(uint16_t* x, const uint16_t* o, const uint16_t* g, const ui
     // With the gate (7 bytes per element) one workgroup per CU stays best.
     const dim3 grid(stream_grid(S, GATE ? 1 : 2)), block(256);
     hipStream_t st = as_stream(stream);
-    if (rows_suit(GATE, true, S, N, R))
+    if (norm_rows_suit(GATE, true, S, N, R))
         return h ? launch_rows<GATE, 2>(x, o, g, w, ridx, s1, sh, h, S, (int)N, (int)R, eps, H3MI_RSQRT_HW, nullptr,
                                         nullptr, q, qs, st, name)
                  : launch_rows<GATE, 1>(x, o, g, w, ridx, s1, sh, h, S, (int)N, (int)R, eps, H3MI_RSQRT_HW, nullptr,
@@ -1662,10 +1639,7 @@ extern "C" int h3mi_gate_bf16(uint16_t* x, const uint16_t* o, const uint16_t* g,
     if (overlap(o, xb, x, xb)) return fail(H3MI_EALIAS, "gate: o overlaps x");
     if (overlap(g, static_cast<size_t>(R) * N * 2, x, xb)) return fail(H3MI_EALIAS, "gate: g overlaps x");
     const int ch = stream_ch(static_cast<int>(N));
-    // One row per workgroup, except over one table row for wide rows that come
-    // from memory: 19200 x 5376 107 against 102 us for the stream, 4800 x 5376 25
-    // against 30, 19200 x 3072 63 against 75.
-    if (ch > 0 && (R > 1 || N <= 4096 || S * N <= int64_t{40} << 20)) {
+    if (ch > 0 && gate_rows_suit(S, N, R)) {
         const int it = static_cast<int>((N + 2047) / 2048);
         const dim3 grid(static_cast<unsigned>(S)), block(256);
 #define H3MI_GATE_ROW_LAUNCH(I)                                                                               \

@@ -54,3 +54,27 @@ def test_streams_and_rows_agree(S, N, R):
         assert torch.equal(t.contiguous().view(torch.uint8), ref.contiguous().view(torch.uint8)), k
     if R > 1:  # out-of-range rows keep the fill and x
         assert bool((whole[0][S // 2] == 3).all()) and torch.equal(whole[5][S // 2], x[S // 2])
+
+
+@pytest.mark.parametrize("R", [1, 5])
+def test_more_rows_than_workgroups_of_one_launch(R):
+    """2^24 + 5 narrow rows: a workgroup of 256 threads each would be more than 2^32 threads."""
+    import h3mi as h
+    S, N, tail = (1 << 24) + 5, 8, 4096
+    print(f"[routes] S={S} N={N} R={R}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x, o = (torch.randn(S, N, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    w, s1, sh, gt = (torch.randn(r, N, generator=g, device="cuda").to(torch.bfloat16) for r in (1, R, R, R))
+    w = w.reshape(-1)
+    ridx = (torch.arange(S, device="cuda") * R // S).to(torch.int32)
+
+    def calls(x, o, ridx):
+        a, b, c = x.clone(), x.clone(), x.clone()
+        return [h.norm_mod(x, w, EPS, ridx, s1, sh), h.gate_norm_mod_(a, o, gt, w, EPS, ridx, s1, sh), a,
+                *h.norm_mod_q(x, w, EPS, ridx, s1, sh), *h.gate_norm_mod_q_(b, o, gt, w, EPS, ridx, s1, sh), b,
+                h.gate_(c, o, gt, ridx)]
+
+    whole = calls(x, o, ridx)
+    for part in (slice(0, tail), slice(S - tail, S)):
+        for k, (a, b) in enumerate(zip(whole, calls(x[part].contiguous(), o[part].contiguous(), ridx[part].contiguous()))):
+            assert torch.equal(a[part].contiguous().view(torch.uint8), b.view(torch.uint8)), (k, part)
