@@ -41,3 +41,24 @@ def test_no_workgroup_per_row_past_the_launch_limit(routes, op, N, R):
     """2^24 workgroups of 256 threads are 2^32 threads, which HIP refuses."""
     for S in (1 << 24, (1 << 24) + 1, (1 << 31) - 1):
         assert not routes(op, S, N, R)
+
+
+@pytest.mark.parametrize("op,S,N,R,rows", [
+    # (route of the faster side as measured: rows = one row per workgroup)
+    ("norm_mod", 4800, 2048, 1, True), ("norm_mod", 9600, 512, 1, False), ("norm_mod", 9600, 3072, 1, False),
+    ("norm_mod", 38400, 512, 2, True), ("norm_mod", 38400, 5376, 2, False), ("norm_mod", 38400, 5120, 5, True),
+    ("norm_mod_q", 3600, 5376, 1, True), ("norm_mod_q", 4600, 5376, 1, False), ("norm_mod_q", 2400, 8192, 1, True),
+    ("norm_mod_q", 4800, 512, 2, True), ("norm_mod_q", 9600, 512, 2, False), ("norm_mod_q", 38400, 128, 5, False),
+    ("norm_mod_q", 19200, 1024, 2, False), ("norm_mod_q", 200000, 64, 2, False), ("norm_mod_q", 14400, 2048, 2, True),
+    ("norm_mod_q", 7200, 5376, 2, False), ("norm_mod_q", 3000, 8192, 5, True),
+    ("gate_norm_mod_", 38400, 1024, 1, True), ("gate_norm_mod_", 38400, 1536, 1, False),
+    ("gate_norm_mod_", 4800, 1536, 1, True), ("gate_norm_mod_", 28800, 1032, 2, False),
+    ("gate_norm_mod_", 19200, 2560, 2, False), ("gate_norm_mod_", 7200, 2560, 2, True),
+    ("gate_norm_mod_", 38400, 5376, 2, True), ("gate_norm_mod_", 38400, 512, 2, True),
+    ("gate_norm_mod_q_", 19200, 3072, 2, False), ("gate_norm_mod_q_", 9600, 3072, 2, True),
+    ("gate_norm_mod_q_", 28800, 3584, 2, False), ("gate_norm_mod_q_", 38400, 512, 2, True),
+    ("gate_norm_mod_q_", 19200, 5376, 5, True), ("gate_norm_mod_q_", 9600, 512, 1, False),
+    ("gate_", 38400, 4096, 1, True), ("gate_", 19200, 5376, 1, False), ("gate_", 38400, 5376, 2, True),
+])
+def test_route_of_the_faster_side(routes, op, S, N, R, rows):
+    assert routes(op, S, N, R) == rows
