@@ -219,8 +219,37 @@ __device__ __forceinline__ uint32_t quant4b(float e0, float e1, float e2, float 
     return pack_low_bytes(__float_as_uint(n[0]), __float_as_uint(n[1]), __float_as_uint(n[2]), __float_as_uint(n[3]));
 }
 
+// Eight elements under one branch: as two calls of quant4b the per-token
+// quantizer was 2-7% slower below 2000 rows (512 x 7168 4.9 against 5.2 us) and
+// the quantizing row streams 1-4%.
 __device__ __forceinline__ uint2 quant8b(const float (&e)[8], float sc, float r, bool exact) {
-    return make_uint2(quant4b(e[0], e[1], e[2], e[3], sc, r, exact), quant4b(e[4], e[5], e[6], e[7], sc, r, exact));
+#pragma clang fp contract(off)
+    float n[8];
+    if (exact) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float q0 = e[j] * r;
+            const float rem = __builtin_fmaf(-q0, sc, e[j]);
+            n[j] = __builtin_fmaf(rem, r, q0);
+        }
+        // the magic add writes its low byte straight into place
+        const float mg = kQuantMagic;
+        uint32_t lo, hi;
+        add_low_byte<0>(lo, n[0], mg);
+        add_low_byte<1>(lo, n[1], mg);
+        add_low_byte<2>(lo, n[2], mg);
+        add_low_byte<3>(lo, n[3], mg);
+        add_low_byte<0>(hi, n[4], mg);
+        add_low_byte<1>(hi, n[5], mg);
+        add_low_byte<2>(hi, n[6], mg);
+        add_low_byte<3>(hi, n[7], mg);
+        return make_uint2(lo, hi);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) n[j] = fminf(fmaxf(rintf(e[j] / sc), -127.0f), 127.0f) + kQuantMagic;
+    }
+    return make_uint2(pack_low_bytes(__float_as_uint(n[0]), __float_as_uint(n[1]), __float_as_uint(n[2]), __float_as_uint(n[3])),
+                      pack_low_bytes(__float_as_uint(n[4]), __float_as_uint(n[5]), __float_as_uint(n[6]), __float_as_uint(n[7])));
 }
 
 // quant8b of 8 packed bf16 values (2 per word).
