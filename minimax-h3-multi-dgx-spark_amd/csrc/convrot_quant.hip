@@ -60,6 +60,7 @@
 #include <vector>
 
 #include "common.h"
+#include "convrot_shape.h"
 
 namespace h3mi {
 namespace {
@@ -395,7 +396,6 @@ constexpr std::array<convrot_fn, sizeof...(P)> row_of(std::integer_sequence<int,
 }
 
 constexpr int kMaxP = 8;
-constexpr int kWprs[] = {1, 2, 4, 8};
 
 template <bool SW>
 convrot_fn pick(int P, int WPR) {
@@ -435,32 +435,6 @@ int ensure_silu_table(hipStream_t stream) {
     return ok();
 }
 
-// Waves per row and passes per wave for a row of `chunks` 1024-element
-// chunks.  Measured at 19200 rows: the registers of more than 3 passes (4 with
-// SwiGLU, whose per-element work is larger) cost more occupancy than the
-// extra waves' reductions cost, and workgroups of 3, 6 or 7 waves schedule
-// worse than 4 or 8 (7 waves x 1 pass at K = 7168, every lane busy: 84.6
-// against 74.9 us for 4 x 2 with one pass slot in 8 empty).  So: the fewest wasted pass slots with at most that many
-// passes, ties to fewer waves per row; past 8 waves, 8 waves and more passes.
-// Few rows (up to 6 a CU, 1.5 with SwiGLU, whose waves each wait for the
-// workgroup's copy of the table): the fewest passes that 8 waves allow, since a
-// wave's passes are a serial chain while most of the chip is idle.  Before ->
-// after: K = 5376 37 rows 5.4 -> 4.0 us, 512 6.4 -> 5.4, 1024 8.2 -> 7.5 (2401
-// 13.1 -> 13.7); SwiGLU K = 5376 128 rows 7.2 -> 5.6 (512 8.5 -> 8.9), K = 14336
-// 37 rows 7.8 -> 6.9.
-void shape_for(int chunks, bool swiglu, int64_t rows, int* wpr, int* passes) {
-    const bool few = rows <= static_cast<int64_t>(cu_count()) * (swiglu ? 3 : 12) / 2;
-    const int pmax = few ? (chunks + 7) / 8 : swiglu ? 4 : 3;
-    int best_w = 8, best_p = (chunks + 7) / 8, best_slots = 1 << 30;
-    for (int w : kWprs) {
-        const int p = (chunks + w - 1) / w;
-        if (p > pmax) continue;
-        if (p * w < best_slots) best_w = w, best_p = p, best_slots = p * w;
-    }
-    *wpr = best_w;
-    *passes = best_p;
-}
-
 }  // namespace
 }  // namespace h3mi
 
@@ -485,7 +459,7 @@ extern "C" int h3mi_quant_convrot_i8(const uint16_t* x, int8_t* q, float* s, int
         return fail(H3MI_EALIAS, "convrot: q, s and x must not overlap");
     const int chunks = static_cast<int>(K / 1024 + (K % 1024 ? 1 : 0));
     int wpr = 1, P = 1;
-    shape_for(chunks, act == H3MI_ACT_SWIGLU, M, &wpr, &P);
+    convrot_shape(chunks, act == H3MI_ACT_SWIGLU, M, cu_count(), &wpr, &P);
     const convrot_fn fn = act == H3MI_ACT_SWIGLU ? pick<true>(P, wpr) : pick<false>(P, wpr);
     if (!fn) return fail(H3MI_EINVAL, "convrot: no kernel for K=%lld", (long long)K);
     const int rpb = rows_per_block(wpr);
