@@ -70,23 +70,29 @@ __device__ __forceinline__ float butterfly(float v) {
 // One wave handles NIT sets of 64 / LPR rows; every load of the wave is
 // issued before the first row is reduced, so a wave keeps NIT x 1 KiB of rows
 // in flight.  Branches around memory operations make the compiler drain all
-// loads at the join, so a row past the end loads row 0 instead (unused) and
+// loads at the join, so a row past the end loads the workgroup's first row instead (unused) and
 // only the stores test the row.  RSTD (the per-row rstd output) is for tests;
-// ROPE: 0 no rotation (rot = 0), 2 full rotation (rot = D), 1 partial; RN
+// ROPE: 0 no rotation (rot = 0), 2 full rotation (rot = D), 1 partial, 3 partial
+// with the partner 8 lanes away (rot = 128, D = 256); RN
 // selects the correctly rounded rsqrt (else the hardware one, as eager).
 //
 // The weights (q's then k's) and the table rows of the workgroup's tokens are
 // staged in LDS as fp32, the table as four planes of rot/2 coefficients per
 // token (R00, R01, R10, R11), so a lane takes its eight pairs' two coefficients
-// as four 16-byte reads, ready to multiply.  Loaded per row instead, each
+// as four 16-byte reads, ready to multiply.  Four floats between the planes put
+// the lower and the upper lanes' reads, 32 bytes apart within a plane, on
+// different banks (12 heads of 256 with rot = 128, 2401 tokens 16.3 -> 14.7 us,
+// 9600 46.3 -> 43.0).  Loaded per row instead, each
 // lane's own eight table words, a wave held 32 registers of them and fetched
 // each table line eight times (and one way or the other waited for them before
-// the next set's rows went out).  The reduction and, at a full rotation of 16
-// lanes, the partner's value are DPP sources; over the LDS crossbar their
-// latency showed (19200 tokens of 56 x 128 196 against 182 us).  With the one
-// launch for every row count (the rest of the rows was a second, guarded one),
-// tokens of 56 x 128, before -> after: 37 10.1 -> 4.0 us, 512 9.6 -> 7.2, 2401 33
-// -> 25.9, 19200 187 -> 182 (6.1 TB/s: memory).
+// the next set's rows went out).  The reduction and, where the partner is 8 lanes
+// away, its value are DPP sources; over the LDS crossbar their latency showed
+// (19200 tokens of 56 x 128 196 against 182 us; 12 heads of 256 with rot = 128,
+// 2401 tokens 14.7 against 14.2).  With the one launch for every row count (the
+// rest of the rows was a second, guarded one), before -> after: 56 x 128 37 tokens
+// 11.1 -> 3.2 us, 512 8.9 -> 7.5, 2401 32.9 -> 26.4; 12 x 256 with rot = 128, 2401
+// tokens 20.0 -> 14.1; long launches, bound by memory (56 x 128 19200 tokens 181
+// us, 6.1 TB/s), the same within 2%.
 template <int LPR, int NIT, bool RSTD, int ROPE, bool RN>
 __global__ __launch_bounds__(256) void rms_rope_kernel(uint16_t* __restrict__ q, uint16_t* __restrict__ k,
                                                        const uint16_t* __restrict__ tab,
@@ -110,7 +116,7 @@ __global__ __launch_bounds__(256) void rms_rope_kernel(uint16_t* __restrict__ q,
     const uint32_t tok0 = per_tok(block0);  // uniform: the workgroup's first token
     // rotation: lanes [0, rot/16) of a row hold the first halves, [rot/16,
     // rot/8) the second halves, the partner lane rot/16 away
-    const int hl = rot / 16, half = rot / 2;
+    const int hl = rot / 16, half = rot / 2, plane = half + 4;  // floats from one plane to the next
     const bool lower = sub < hl;
     const bool rotated = ROPE == 2 || sub < 2 * hl;
     const int src = rotated ? (lower ? lane + hl : lane - hl) : lane;
@@ -149,11 +155,11 @@ __global__ __launch_bounds__(256) void rms_rope_kernel(uint16_t* __restrict__ q,
     wsh[D + wt] = bf16_f32(wk1);
     if constexpr (ROPE > 0) {
         auto stage = [&](int p, uint2 w) {
-            float* const d = tsh + (p / half) * 4 * half + p % half;
+            float* const d = tsh + (p / half) * 4 * plane + p % half;
             d[0] = bf16_lo(w.x);
-            d[half] = bf16_hi(w.x);
-            d[2 * half] = bf16_lo(w.y);
-            d[3 * half] = bf16_hi(w.y);
+            d[plane] = bf16_hi(w.x);
+            d[2 * plane] = bf16_lo(w.y);
+            d[3 * plane] = bf16_hi(w.y);
         };
         if (static_cast<int>(threadIdx.x) < pairs) stage(threadIdx.x, t0);
         for (int p = threadIdx.x + 256; p < pairs; p += 256) stage(p, pt[p]);  // few heads: many tokens
@@ -206,9 +212,9 @@ __global__ __launch_bounds__(256) void rms_rope_kernel(uint16_t* __restrict__ q,
         if constexpr (ROPE > 0) {
             // lower lane: out = R00 y + R01 p; upper lane: R10 p + R11 y, the
             // same sum in the other order
-            const float* tr = tsh + rel[it] * 4 * half + pair0;
-            const float* const po_ = tr + (lower ? 0 : 3 * half);
-            const float* const pp_ = tr + (lower ? half : 2 * half);
+            const float* tr = tsh + rel[it] * 4 * plane + pair0;
+            const float* const po_ = tr + (lower ? 0 : 3 * plane);
+            const float* const pp_ = tr + (lower ? plane : 2 * plane);
             const float4 o0 = *reinterpret_cast<const float4*>(po_), o1 = *reinterpret_cast<const float4*>(po_ + 4);
             const float4 q0 = *reinterpret_cast<const float4*>(pp_), q1 = *reinterpret_cast<const float4*>(pp_ + 4);
             const float co[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
@@ -216,7 +222,7 @@ __global__ __launch_bounds__(256) void rms_rope_kernel(uint16_t* __restrict__ q,
             float p[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                if constexpr (ROPE == 2 && LPR == 16) p[i] = dpp_xor<8>(y[i]);  // rot / 16 lanes apart
+                if constexpr (ROPE == 3 || (ROPE == 2 && LPR == 16)) p[i] = dpp_xor<8>(y[i]);  // rot / 16 = 8 lanes apart
                 else p[i] = __shfl(y[i], src, 64);
             }
 #pragma unroll
@@ -290,12 +296,12 @@ extern "C" int h3mi_rms_rope_split_half_bf16(uint16_t* q, uint16_t* k, const uin
         const unsigned blocks = static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block);
         // the weights, and the table rows of as many tokens as a workgroup's rows can touch
         const int64_t toks = (rows_per_block - 2) / (2 * H) + 2;
-        size_t lds = static_cast<size_t>(2 * D + (rot ? toks * 2 * rot : 0)) * sizeof(float);
+        size_t lds = static_cast<size_t>(2 * D + (rot ? toks * 4 * (rot / 2 + 4) : 0)) * sizeof(float);
         // Rows that come from memory stream faster with five workgroups per CU
         // than with the seven that the registers allow, so the LDS of a long
-        // launch is padded: 19200 tokens of 56 x 128 182 against 187 us, 40 x 128
-        // 133.5 against 141, 2401 of 56 25.9 against 26.4; 1024 (29 MB) 13.1
-        // against 12.3.
+        // launch is padded: 19200 tokens of 56 x 128 181.5 against 187.5 us, 40 x 128
+        // 136.1 against 142.8, 12 x 256 79.8 against 81.4, 9600 of 56 x 128 91.5
+        // against 93.9.
         if (rows * D * 2 >= int64_t{48} << 20 && lds < 32768) lds = 32768;
         hipLaunchKernelGGL((rms_rope_kernel<L, NIT, R, P, N>), dim3(blocks), dim3(256), lds, as_stream(stream), q, k, tab,
                            qw, kw, static_cast<int>(S), static_cast<int>(H), per_tok, ldq, ldk, static_cast<int>(rot), eps,
@@ -314,7 +320,11 @@ extern "C" int h3mi_rms_rope_split_half_bf16(uint16_t* q, uint16_t* k, const uin
     using R0 = std::integral_constant<int, 0>;
     using R1 = std::integral_constant<int, 1>;
     using R2 = std::integral_constant<int, 2>;
+    using R3 = std::integral_constant<int, 3>;
     auto run1 = [&](auto lpr_c, auto rstd_c) {
+        if constexpr (decltype(lpr_c)::value == 32) {
+            if (rot == 128) return run2(lpr_c, rstd_c, R3{});
+        }
         if (rot == D) run2(lpr_c, rstd_c, R2{});
         else if (rot) run2(lpr_c, rstd_c, R1{});
         else run2(lpr_c, rstd_c, R0{});

@@ -169,3 +169,9 @@ def test_rest_rows_and_many_tokens_match_eager_and_oracle(S, H, D, rot):
     """Row counts that leave a part of a workgroup, in launches of four and of
     two row sets per wave, and workgroups whose rows span many tokens."""
     test_matches_eager_and_oracle(S, H, D, rot)
+
+
+@pytest.mark.parametrize("S,H", [(1801, 12), (65, 1), (37, 24)])
+def test_partner_eight_lanes_away_in_a_row_of_32(S, H):
+    """rot = 128 of 256: half of a row's lanes rotate, with the DPP partner."""
+    test_matches_eager_and_oracle(S, H, 256, 128)
