@@ -238,6 +238,12 @@ __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+template <bool CACHED, class V>
+__device__ __forceinline__ void store_out(V v, V* p) {
+    if constexpr (CACHED) *p = v;
+    else __builtin_nontemporal_store(v, p);
+}
+
 // LDS-staged epilogue for the bf16 output, one 32-row x 64-column slab
 // (4 KiB of bf16) at a time through a private 4 KiB LDS buffer per wave.
 //   * Scales: the workgroup's ws, bias and xs slices were copied into LDS
@@ -252,12 +258,13 @@ __device__ __forceinline__ void static_for(F&& f) {
 //     (chunk c sits at c ^ (key >> 1), its 8-byte halves swapped when key is
 //     odd), and each row leaves as 128 contiguous bytes with non-temporal
 //     stores (the output is never re-read, so it should not displace
-//     operand panels from L2).  In a full tile a store's address is a
+//     operand panels from L2), or, with CACHED, through the cache (see
+//     gemm_entry).  In a full tile a store's address is a
 //     wave-uniform 64-bit base (scalar registers) plus the lane's fixed
 //     32-bit byte offset: one 64-bit add per store.
 // One wave reads back only what it wrote, and LDS operations of one wave
 // complete in order, so no barrier is needed between slabs.
-template <class T, bool BIAS, bool FULL, int JB = 0, int JE = T::FM>
+template <class T, bool CACHED, bool BIAS, bool FULL, int JB = 0, int JE = T::FM>
 __device__ __forceinline__ void store_tile_lds_impl(const v16i (&acc)[T::FN][T::FM], const uint8_t* sc,
                                                     uint16_t* __restrict__ out, int M, int N, int64_t ldo, int m0, int n0,
                                                     int wm, int wn, int lane, uint8_t* wbuf) {
@@ -345,47 +352,35 @@ __device__ __forceinline__ void store_tile_lds_impl(const v16i (&acc)[T::FN][T::
                 if (key & 1) v = v4u{v[2], v[3], v[0], v[1]};
                 if constexpr (FULL) {
                     uint16_t* row = out + static_cast<int64_t>(mb + j * 32 + q * 8) * ldo + nb + sl * 64;
-                    __builtin_nontemporal_store(v, reinterpret_cast<v4u*>(reinterpret_cast<char*>(row) + lane_off));
+                    store_out<CACHED>(v, reinterpret_cast<v4u*>(reinterpret_cast<char*>(row) + lane_off));
                     continue;
                 }
                 const int m = mb + j * 32 + r;
                 const int n = nb + sl * 64 + c * 8;
                 uint16_t* o = out + static_cast<int64_t>(m) * ldo + n;
                 if (m < M && n < N) {
-                    if (n + 8 <= N) {
-                        // cached: see store_tile_lds (A1 tiles get whole-line rows)
-                        if constexpr (T::A1) __builtin_nontemporal_store(v, reinterpret_cast<v4u*>(o));
-                        else *reinterpret_cast<v4u*>(o) = v;
-                    } else {  // N % 4 == 0: the row ends half-way through this chunk
-                        __builtin_nontemporal_store(v2u{v[0], v[1]}, reinterpret_cast<v2u*>(o));
-                    }
+                    if (n + 8 <= N) store_out<CACHED>(v, reinterpret_cast<v4u*>(o));
+                    else store_out<CACHED>(v2u{v[0], v[1]}, reinterpret_cast<v2u*>(o));  // N % 4 == 0: half a chunk
                 }
             }
         }
     });
 }
 
-template <class T, int JB = 0, int JE = T::FM>
+template <class T, bool CACHED, int JB = 0, int JE = T::FM>
 __device__ __forceinline__ void store_tile_lds(const v16i (&acc)[T::FN][T::FM], const uint8_t* sc, bool has_bias,
                                                uint16_t* __restrict__ out, int M, int N, int64_t ldo, int m0, int n0,
                                                int wm, int wn, int lane, uint8_t* wbuf) {
     // Uniform branches around the whole epilogue, none inside it: bias or
     // not, and whether the workgroup tile lies wholly inside the output (and
     // eight output rows span under 2^31 bytes, so lane offsets fit 32 bits).
-    // Rows that do not start on a 128-byte line (N = 9000) take the bounds-checked
-    // variant too, whose stores are cached: a slab's segment of a row ends inside
-    // two lines whose other parts the neighbouring slabs write, and non-temporal
-    // stores sent each part to memory by itself; the L2 joins them (10000 x 9000
-    // x 384 69 against 108 us, x 1536 147 against 167).  A copy of the unchecked
-    // variant with cached stores cost the other shapes 1% by its size alone.
-    const bool lines = T::A1 || ((ldo & 63) == 0 && (reinterpret_cast<uintptr_t>(out) & 127) == 0);
-    const bool full = lines && m0 + T::BM <= M && n0 + T::BN <= N && ldo < (int64_t{1} << 27);
+    const bool full = m0 + T::BM <= M && n0 + T::BN <= N && ldo < (int64_t{1} << 27);
     if (has_bias) {
-        if (full) store_tile_lds_impl<T, true, true, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
-        else store_tile_lds_impl<T, true, false, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
+        if (full) store_tile_lds_impl<T, CACHED, true, true, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
+        else store_tile_lds_impl<T, CACHED, true, false, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
     } else {
-        if (full) store_tile_lds_impl<T, false, true, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
-        else store_tile_lds_impl<T, false, false, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
+        if (full) store_tile_lds_impl<T, CACHED, false, true, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
+        else store_tile_lds_impl<T, CACHED, false, false, JB, JE>(acc, sc, out, M, N, ldo, m0, n0, wm, wn, lane, wbuf);
     }
 }
 
@@ -394,7 +389,11 @@ __device__ __forceinline__ void store_tile_lds(const v16i (&acc)[T::FN][T::FM], 
 // ws[n0 .. n0+BN), wave 1 xs[m0 .. m0+BM), wave 2 bias[n0 .. n0+BNB) (the
 // entries past BN are copied and never read).  Entries past N or M are out of
 // the buffer range and read as zero.
-template <class T>
+// CACHED: a copy for each of the two bf16 kernels, as for widen_bias.  Shared by
+// them, these helpers were optimized without their one caller's pointers, which
+// left null checks of the LDS addresses and 10 more spilled scalar registers in
+// the 256x256 kernel (4799 x 5376 x 7168 1% slower).
+template <class T, bool CACHED>
 __device__ __forceinline__ void issue_scales(const float* xs, const float* ws, const uint16_t* bias, int M, int N, int m0,
                                              int n0, int lane, int wid, uint8_t* sc) {
     static_assert(T::NW >= 3 && T::BN % 64 == 0 && T::BM % 64 == 0, "scale copy layout");
@@ -419,7 +418,7 @@ __device__ __forceinline__ void issue_scales(const float* xs, const float* ws, c
 
 // The copying wave widens the bias slice at sc + SC_B16 (bf16) into f32 at
 // sc + SC_B32, once per tile, after its copy has landed.
-template <class T>
+template <class T, bool CACHED>
 __device__ __forceinline__ void widen_bias(uint8_t* sc, int lane) {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(sc + T::SC_B16);
     float2* dst = reinterpret_cast<float2*>(sc + T::SC_B32);
@@ -430,7 +429,7 @@ __device__ __forceinline__ void widen_bias(uint8_t* sc, int lane) {
     }
 }
 
-template <class T, bool OUT_I32>
+template <class T, bool OUT_I32, bool CACHED = false>
 __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WPE, T::WPE))) void w8a8_gemm_direct_kernel(
     const int8_t* __restrict__ X, const int8_t* __restrict__ W, const float* __restrict__ xs,
     const float* __restrict__ ws, const uint16_t* __restrict__ bias, void* __restrict__ out, int M, int N, int K,
@@ -728,7 +727,7 @@ __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WPE, T
         // can join the loads in flight without disturbing the vmcnt counts.
         const int cur = (KT - 1 + base) & 1, fr = cur ^ 1;
         uint8_t* const sc = SC_IN_RING ? lds + fr * T::SSTAGE + T::SSTAGE - SC_BYTES : lds + LDS_BYTES;
-        if constexpr (STAGED) issue_scales<T>(xs, ws, bias, M, N, m0, n0, lane, wid, sc);
+        if constexpr (STAGED) issue_scales<T, CACHED>(xs, ws, bias, M, N, m0, n0, lane, wid, sc);
         static_for<T::KS>([&](auto ks_c) {
             constexpr int ks = decltype(ks_c)::value;
             constexpr int slot = ks & 1;
@@ -744,7 +743,7 @@ __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WPE, T
             if constexpr (STAGED) {
                 wait_vm<0>();  // this wave's scale copy has landed
                 if (wid == 2 && bias) {
-                    widen_bias<T>(sc, lane);
+                    widen_bias<T, CACHED>(sc, lane);
                     wait_lgkm0();  // the widened bias is in LDS before the barrier
                 }
             }
@@ -801,7 +800,7 @@ __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WPE, T
                             for (int r = 0; r < 4; ++r) acc[i][KB + jj][4 * q + r] += p[r];
                         }
                 if constexpr (STAGED) {
-                    store_tile_lds<T, KB, KB + FMH>(acc, sc, bias != nullptr, static_cast<uint16_t*>(out), M, N, ldo,
+                    store_tile_lds<T, CACHED, KB, KB + FMH>(acc, sc, bias != nullptr, static_cast<uint16_t*>(out), M, N, ldo,
                                                      m0, n0, wm, wn, lane, lds + fr * T::SSTAGE + wid * 4096);
                 } else {
                     store_tile<T, OUT_I32, KB, KB + FMH>(acc, xs, ws, bias, out, M, N, ldo, m0, n0, wm, wn, lr, lk);
@@ -810,7 +809,7 @@ __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WPE, T
             if (grp == 0) swap_halves(std::integral_constant<int, 0>{});
             else swap_halves(std::integral_constant<int, 1>{});
         } else if constexpr (STAGED) {
-            store_tile_lds<T>(acc, sc, bias != nullptr, static_cast<uint16_t*>(out), M, N, ldo, m0, n0, wm, wn, lane,
+            store_tile_lds<T, CACHED>(acc, sc, bias != nullptr, static_cast<uint16_t*>(out), M, N, ldo, m0, n0, wm, wn, lane,
                               lds + fr * T::SSTAGE + wl * 4096);
         } else {
             store_tile<T, OUT_I32>(acc, xs, ws, bias, out, M, N, ldo, m0, n0, wm, wn, lr, lk);
@@ -896,22 +895,31 @@ struct Config {
     const char* name;
     int bm, bn, kmul, threads;  // kmul: K must be a multiple of it (BK, times the K-groups)
     kernel_fn bf16_kernel;
+    kernel_fn bf16_cached;  // its output stored through the cache; null where there is no such variant
     kernel_fn i32_kernel;
     bool resident;  // grid of resident workgroups looping over the tiles (else one workgroup per tile)
 };
 
+// The A1 tilings have no registers for the cached epilogue (116 against 56
+// spilled) and 128x128 tiles are faster without (gemm_entry).
+template <class T>
+constexpr kernel_fn cached_kernel() {
+    if constexpr (T::A1 || T::BM * T::BN <= 128 * 128) return nullptr;
+    else return w8a8_gemm_direct_kernel<T, false, true>;
+}
+
 #define H3MI_DCFG(NAME, T)                                                                                      \
     {NAME, T::BM, T::BN, T::BK * T::SPLITK, T::NT, w8a8_gemm_direct_kernel<T, false>,                         \
-     w8a8_gemm_direct_kernel<T, true>, false}
+     cached_kernel<T>(), w8a8_gemm_direct_kernel<T, true>, false}
 // Resident grids: one tile per workgroup at a time, so no split-K tiling.
 #define H3MI_RCFG(NAME, T)                                                                                      \
     {NAME, T::BM, T::BN, T::BK + 0 * sizeof(char[T::SPLITK == 1 ? 1 : -1]), T::NT,                             \
-     w8a8_gemm_direct_kernel<T, false>, w8a8_gemm_direct_kernel<T, true>, true}
+     w8a8_gemm_direct_kernel<T, false>, cached_kernel<T>(), w8a8_gemm_direct_kernel<T, true>, true}
 
 // Wave-split tiles (gemm_kwave.h): KTile<MF, NF> is 16 MF rows of X by 16 NF of W.
 #define H3MI_KCFG(NAME, ...) \
     {NAME, KTile<__VA_ARGS__>::BM, KTile<__VA_ARGS__>::BN, 128, KTile<__VA_ARGS__>::NT, \
-     w8a8_gemm_kwave_kernel<KTile<__VA_ARGS__>, false>, w8a8_gemm_kwave_kernel<KTile<__VA_ARGS__>, true>, false}
+     w8a8_gemm_kwave_kernel<KTile<__VA_ARGS__>, false>, nullptr, w8a8_gemm_kwave_kernel<KTile<__VA_ARGS__>, true>, false}
 
 const Config kConfigs[] = {
     H3MI_DCFG("d_bm256_bn256_bk128_s2_g4_w8m_st1", D256w8st1),
@@ -1156,7 +1164,18 @@ int gemm_entry(const int8_t* xq, const int8_t* w, const float* xs, const float* 
     const int tiles_m = static_cast<int>((M + c.bm - 1) / c.bm), tiles_n = static_cast<int>((N + c.bn - 1) / c.bn);
     const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
     if (tiles > 0x7FFFFFFF) return fail(H3MI_EINVAL, "%s: too many tiles", name);
-    const kernel_fn fn = OUT_I32 ? c.i32_kernel : c.bf16_kernel;
+    // Output rows that start off 32-byte sectors (N = 9000) are stored through the
+    // cache once the output is past 16 MiB: a slab's segment of a row ends inside
+    // sectors whose other parts the neighbouring slabs write, and non-temporal
+    // stores send each part to memory by itself; the L2 joins them (256x256 tiles,
+    // 10000 x 9000 x 384 110 -> 72 us, 11504 x 1192 x 512 19.8 -> 15.5, 2182 x 12856
+    // x 3072 93 -> 85).  Over 140 shapes: rows on sectors, smaller outputs and
+    // 128x128 tiles were the same or up to 10% faster with non-temporal stores
+    // (2961 x 2336 x 1280 14.3 against 15.8, 8903 x 648 x 896 11.7 against 12.7).
+    // A kernel of its own, so that the others' epilogue stays free of it.
+    const bool sectors = ldo % 16 == 0 && aligned(out, 32);
+    const bool cached = c.bf16_cached && !sectors && M * N > int64_t{8} << 20;
+    const kernel_fn fn = OUT_I32 ? c.i32_kernel : cached ? c.bf16_cached : c.bf16_kernel;
     int64_t grid = tiles;
     if (c.resident) {
         const int64_t cap = static_cast<int64_t>(cu_count()) * resident_per_cu(fn, c.threads);

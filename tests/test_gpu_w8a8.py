@@ -372,3 +372,34 @@ def test_allcfg_autotune_picks_a_config_and_keeps_the_bytes(monkeypatch):
     b = h3mi.int8_mm_scaled(xq, w, xs, ws)
     assert torch.equal(a, ref) and torch.equal(b, ref)
     assert h3mi.config_for(M, N, K) == h3mi.config_for(M, N, K)  # the heuristic is restored after each call
+
+
+@pytest.mark.parametrize("N,ldo,off", [(1000, 1000, 0), (1000, 1028, 0), (1024, 1024, 4), (968, 1024, 0), (1024, 1040, 16)])
+def test_output_rows_off_sectors(N, ldo, off):
+    """Output rows that start off 32-byte sectors (their length, their stride or
+    the first row's address), in an output past the 16 MiB from which they are
+    stored through the cache, and rows on sectors: every configuration writes the
+    exact epilogue's bytes, whole tiles and edges, and nothing beside them."""
+    h = _h3mi()
+    from h3mi._lib import check, lib, ptr, stream_of
+    M, K = 8900, 256
+    g = torch.Generator(device="cuda").manual_seed(N + ldo + off)
+    xq, w = (torch.randint(-127, 128, (r, K), generator=g, device="cuda", dtype=torch.int8) for r in (M, N))
+    xs, ws = (torch.rand(r, generator=g, device="cuda") for r in (M, N))
+    bias = torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)
+    plain = (h.int8_mm_i32(xq, w).float() * xs[:, None]) * ws
+    want = {False: plain.to(torch.bfloat16), True: (plain + bias.float()).to(torch.bfloat16)}
+    try:
+        for name in h.list_configs():
+            print(f"[rows off sectors] {name} N={N} ldo={ldo} off={off}", flush=True)
+            h.set_config(name)
+            for b in (False, True):
+                buf = torch.full((M * ldo + off + 64,), 7, dtype=torch.bfloat16, device="cuda")
+                out = buf[off:]
+                check(lib.h3mi_w8a8_gemm_bf16(ptr(xq), ptr(w), ptr(xs), ptr(ws), ptr(bias) if b else None, ptr(out), M, N, K,
+                                              K, K, ldo, stream_of(xq)))
+                rows = out[:M * ldo].view(M, ldo)
+                assert torch.equal(rows[:, :N], want[b]), (name, b)
+                assert bool((rows[:, N:] == 7).all()) and bool((buf[:off] == 7).all()) and bool((out[M * ldo:] == 7).all())
+    finally:
+        h.set_config("auto")
