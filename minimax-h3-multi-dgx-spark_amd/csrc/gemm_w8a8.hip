@@ -1047,7 +1047,8 @@ int wave_split_or(int other, int64_t M, int64_t N, int64_t K, int64_t cus) {
 // the smaller grids, one of the 128x128, 128x192 or larger tiles is picked by
 // whole rounds over the CUs times tile area and then weighed against the
 // wave-split tilings by predicted time.
-int pick_config(int64_t M, int64_t N, int64_t K) {
+// `sectors`: the output's rows start on 32-byte sectors (gemm_entry).
+int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
     {
         // a forced configuration that cannot take this K (split-K tilings
         // need K % 256 == 0) leaves the call to the heuristic
@@ -1072,10 +1073,11 @@ int pick_config(int64_t M, int64_t N, int64_t K) {
     // work per CU: N = 15360 and 5120); with a ragged last column (N = 5376)
     // they measured 3-4% slower than 320x256, so they are offered only then.
     const bool n320 = N % 320 == 0;
-    // 256x384 tiles are offered when output rows start on 128-byte lines: their
-    // epilogue has no room for the cached stores that other rows want
-    // (32768 x 9000 x 5120 1300 against 1208 us, x 768 515 against 306).
-    const bool lines = N % 64 == 0;
+    // 256x384 tiles are offered when output rows start on sectors: their epilogue
+    // has no room for the cached stores that other rows want (32768 x 9000 x 5120
+    // 1300 against 1208 us, x 768 515 against 306).  On sectors off 128-byte
+    // lines they stay ahead where the rounds say so (16000 x 5408 x 5120 364
+    // against 374, 16000 x 10272 x 3072 421 against 437).
     const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
     if (t256 < 2 * cus) {
         // Fewer than two 256x256 tiles per CU: 128x128 tiles (two workgroups
@@ -1102,7 +1104,7 @@ int pick_config(int64_t M, int64_t N, int64_t K) {
         // 768 x 28672 x 5376 110 against 138 us, 1536 x 15360 x 5120 98 against
         // 116, 4096 x 5376 x 14336 260 against 327; with a short K its epilogue
         // weighs more (2400 x 9000 x 1536: 58.6 against 53.3).
-        const double c384 = lines && K >= 3072 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
+        const double c384 = sectors && K >= 3072 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
         const double ck2 = K % 256 == 0 ? rounds(128, 192) * 128.0 * 192.0 / 0.88 : 1e300;
         int c = c256 < c128 ? big : small;
         if (ck2 < c256 && ck2 < c128) c = split;
@@ -1122,7 +1124,7 @@ int pick_config(int64_t M, int64_t N, int64_t K) {
     // areas alone, which sent short K to 256x384 tiles (10000 x 13824 x 384 110
     // against 88 us, 32768 x 13824 x 768 439 against 383).
     const double w256 = rounds(256, 256) * 256.0 * 256.0 * (K + 554);
-    const double w384 = lines ? rounds(256, 384) * 256.0 * 384.0 * (K + 820) / 1.07 : 1e300;
+    const double w384 = sectors ? rounds(256, 384) * 256.0 * 384.0 * (K + 820) / 1.07 : 1e300;
     const double w320 = rounds(320, 256) * 320.0 * 256.0 * (K + 541);
     const double w320n = n320 ? rounds(256, 320) * 256.0 * 320.0 * (K + 640) / 1.024 : 1e300;
     if (w320n < w256 && w320n < w384 && w320n < w320) return flat;
@@ -1160,7 +1162,8 @@ int gemm_entry(const int8_t* xq, const int8_t* w, const float* xs, const float* 
     const size_t ob = static_cast<size_t>(M) * ldo * (OUT_I32 ? 4 : 2);
     if (overlap(out, ob, xq, static_cast<size_t>(M) * ldx) || overlap(out, ob, w, static_cast<size_t>(N) * ldw))
         return fail(H3MI_EALIAS, "%s: out overlaps an input", name);
-    const Config& c = kConfigs[pick_config(M, N, K)];
+    const bool sectors = ldo % 16 == 0 && aligned(out, 32);
+    const Config& c = kConfigs[pick_config(M, N, K, sectors)];
     const int tiles_m = static_cast<int>((M + c.bm - 1) / c.bm), tiles_n = static_cast<int>((N + c.bn - 1) / c.bn);
     const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
     if (tiles > 0x7FFFFFFF) return fail(H3MI_EINVAL, "%s: too many tiles", name);
@@ -1173,7 +1176,6 @@ int gemm_entry(const int8_t* xq, const int8_t* w, const float* xs, const float* 
     // 128x128 tiles were the same or up to 10% faster with non-temporal stores
     // (2961 x 2336 x 1280 14.3 against 15.8, 8903 x 648 x 896 11.7 against 12.7).
     // A kernel of its own, so that the others' epilogue stays free of it.
-    const bool sectors = ldo % 16 == 0 && aligned(out, 32);
     const bool cached = c.bf16_cached && !sectors && M * N > int64_t{8} << 20;
     const kernel_fn fn = OUT_I32 ? c.i32_kernel : cached ? c.bf16_cached : c.bf16_kernel;
     int64_t grid = tiles;
@@ -1250,7 +1252,7 @@ extern "C" int h3mi_w8a8_gemm_i32(const int8_t* xq, const int8_t* w, int32_t* ac
 
 extern "C" int h3mi_w8a8_config(int64_t M, int64_t N, int64_t K, char* buf, int64_t buflen) {
     if (!buf || buflen <= 0) return fail(H3MI_EINVAL, "w8a8_config: no buffer");
-    const char* nm = kConfigs[pick_config(M, N, K)].name;
+    const char* nm = kConfigs[pick_config(M, N, K, N % 16 == 0)].name;  // a contiguous, aligned output
     strncpy(buf, nm, static_cast<size_t>(buflen - 1));
     buf[buflen - 1] = '\0';
     return ok();

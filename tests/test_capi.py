@@ -246,6 +246,12 @@ def test_heuristic_on_small_grids(M, N, K, tile):
     assert h3mi.config_for(M, N, K) == tile
 
 
+@pytest.mark.parametrize("N,wide", [(10304, True), (10272, True), (10256, True), (10280, False), (10276, False)])
+def test_256x384_tiles_need_output_rows_on_sectors(N, wide):
+    import h3mi
+    assert h3mi.config_for(16000, N, 5120).startswith("d_bm256_bn384") == wide
+
+
 def test_buffer_probe_argument_errors():
     """The range-check probe rejects its arguments before any launch."""
     from h3mi import _lib
