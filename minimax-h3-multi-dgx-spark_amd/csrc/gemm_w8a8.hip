@@ -1102,9 +1102,10 @@ int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
         const double c320 = n320 ? rounds(256, 320) * 256.0 * 320.0 / (1.5 * 1.024) : 1e300;
         // 256x384 (past half a round of 256x256 tiles that would need a second):
         // 768 x 28672 x 5376 110 against 138 us, 1536 x 15360 x 5120 98 against
-        // 116, 4096 x 5376 x 14336 260 against 327; with a short K its epilogue
-        // weighs more (2400 x 9000 x 1536: 58.6 against 53.3).
-        const double c384 = sectors && K >= 3072 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
+        // 116, 4096 x 5376 x 14336 260 against 327, 2400 x 9216 x 1536 39 against 44,
+        // x 768 26.8 against 28.7; at K = 384 its epilogue weighs more (4096 x 5376
+        // 20.3 against 19.9).
+        const double c384 = sectors && K >= 768 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
         const double ck2 = K % 256 == 0 ? rounds(128, 192) * 128.0 * 192.0 / 0.88 : 1e300;
         int c = c256 < c128 ? big : small;
         if (ck2 < c256 && ck2 < c128) c = split;

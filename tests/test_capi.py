@@ -246,6 +246,14 @@ def test_heuristic_on_small_grids(M, N, K, tile):
     assert h3mi.config_for(M, N, K) == tile
 
 
+@pytest.mark.parametrize("M,N,K,wide", [(2400, 9216, 1536, True), (1536, 13824, 768, True), (4096, 5376, 768, True),
+                                        (4096, 5376, 384, False), (768, 28672, 384, False)])
+def test_256x384_tiles_on_small_grids_by_k(M, N, K, wide):
+    """Ahead of the other tilings from K = 768 up where they save a round of tiles."""
+    import h3mi
+    assert h3mi.config_for(M, N, K).startswith("d_bm256_bn384") == wide
+
+
 @pytest.mark.parametrize("N,wide", [(10304, True), (10272, True), (10256, True), (10280, False), (10276, False)])
 def test_256x384_tiles_need_output_rows_on_sectors(N, wide):
     import h3mi
