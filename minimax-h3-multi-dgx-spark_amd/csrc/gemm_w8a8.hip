@@ -1094,7 +1094,8 @@ int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
         // the 128x128 one's work per CU, but at C0 (2048 x 3072) one such tile
         // per CU replaces two 128x128 ones: 24.2 against 27.5 us; the block's
         // cross-attention KV projection (512 x 10240, K = 5120): 34.4 against
-        // 37.2 us.  With more tiles than CUs, or half of them idle, 128x128
+        // 37.2 us; with weights from memory and the quantizer before it 28.5 against
+        // 30.9 and 52.9 against 54.5.  With more tiles than CUs, or half of them idle, 128x128
         // wins (M = 1536, N = K = 4096: 31.5 against 48.2 us).
         const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
         const double c128 = static_cast<double>((t128 + cus - 1) / cus) * 128.0 * 128.0;
@@ -1111,11 +1112,12 @@ int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
         if (ck2 < c256 && ck2 < c128) c = split;
         if (c320 < c256 && c320 < c128 && c320 < ck2) c = flat;
         if (c384 < c256 && c384 < c128 && c384 < ck2 && c384 < c320) c = wide;
-        // One 128x128 tile per CU or fewer: two K-groups of waves instead of one,
-        // from K = 4096 up (768 x 5376 x 14336 66 against 78 us, 128 x 28672 x
-        // 5376 38 against 46, 384 x 10240 x 5120 33.9 against 36.2); shorter K
-        // stays with the plain tile, which the tests name at 1024 x 3072 x 3072.
-        if (c == small && t128 <= cus && K % 256 == 0 && K >= 4096) c = small_k2;
+        // One 128x128 tile per CU or fewer: two K-groups of waves instead of one, from
+        // K = 1024 up, ahead at every one of 13 outputs (142 to 256 tiles) and K to
+        // 5120: 1024 x 3072 x 1024 9.1 against 9.4 us, x 3072 16.7 against 18.8, 768 x
+        // 3072 x 3072 16.5 against 19.2, 384 x 9000 x 1536 11.8 against 12.5, 128 x
+        // 21504 x 3072 26.9 against 28.8.  Even at 768, 1-4% behind at 512.
+        if (c == small && t128 <= cus && K % 256 == 0 && K >= 1024) c = small_k2;
         return wave_split_or(c, M, N, K, cus);
     }
     // Work of the busiest CU: rounds times tile area times K plus what a tile

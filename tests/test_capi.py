@@ -221,12 +221,12 @@ def test_rms_rope_argument_errors():
     (19200, 5376, 14336, "d_bm320_bn256_bk128_s2_g4_w8m_st1_sw_res"),     # H3 fc2
     (2048, 3072, 3072, "d_bm128_bn192_bk128_s2_g8_w2x2_sw_k2"),           # C0: one split-K tile per CU
     (512, 10240, 5120, "d_bm128_bn192_bk128_s2_g8_w2x2_sw_k2"),           # cross-attention KV projection
-    (1024, 3072, 3072, "d_bm128_bn128_bk128_s2_g4_o2"),                   # 192 small tiles
+    (1024, 3072, 3072, "d_bm128_bn128_bk128_s2_g8_w2x2_sw_k2"),           # 192 small tiles: two K-groups 16.7 us, one 18.8
     (1536, 4096, 4096, "d_bm128_bn128_bk128_s2_g4_o2"),                   # 264 split-K tiles: two rounds
     (2048, 3072, 3200, "d_bm128_bn128_bk128_s2_g4_o2"),                   # K % 256 != 0: no split-K
 ])
 def test_heuristic_picks_the_measured_tiling(M, N, K, tile):
-    """The tiling the heuristic picks at the workload shapes, each the winner of a same-process A/B on the box
+    """The tiling the heuristic picks at the workload shapes, each the winner of a same-process A/B
     (the library assumes MI355X's 256 CUs when no GPU is visible, as here)."""
     import h3mi
     assert h3mi.config_for(M, N, K) == tile
@@ -244,6 +244,14 @@ def test_heuristic_picks_the_measured_tiling(M, N, K, tile):
 def test_heuristic_on_small_grids(M, N, K, tile):
     import h3mi
     assert h3mi.config_for(M, N, K) == tile
+
+
+@pytest.mark.parametrize("M,N,K,k2", [(1024, 3072, 1024, True), (768, 3072, 3072, True), (2048, 2048, 2048, True),
+                                      (1024, 3072, 896, False), (1024, 3072, 1152, False)])
+def test_two_k_groups_where_tiles_fit_the_cus(M, N, K, k2):
+    """At most one 128x128 tile per CU, K a multiple of 256 from 1024 up."""
+    import h3mi
+    assert h3mi.config_for(M, N, K) == ("d_bm128_bn128_bk128_s2_g8_w2x2_sw_k2" if k2 else "d_bm128_bn128_bk128_s2_g4_o2")
 
 
 @pytest.mark.parametrize("M,N,K,wide", [(2400, 9216, 1536, True), (1536, 13824, 768, True), (4096, 5376, 768, True),
