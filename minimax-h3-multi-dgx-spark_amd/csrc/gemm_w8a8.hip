@@ -1118,7 +1118,11 @@ int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
         // 3072 x 3072 16.5 against 19.2, 384 x 9000 x 1536 11.8 against 12.5, 128 x
         // 21504 x 3072 26.9 against 28.8.  Even at 768, 1-4% behind at 512.
         if (c == small && t128 <= cus && K % 256 == 0 && K >= 1024) c = small_k2;
-        return wave_split_or(c, M, N, K, cus);
+        // More 128x128 tiles than CUs: those run two to a CU, faster together than
+        // the model's one after the other, and were ahead of the wave-split pick on
+        // 37 of 38 outputs of 260 to 364 tiles (671 x 6312 x 4992 38.7 against 53.8
+        // us, 7714 x 616 x 10624 75 against 104; the other equal).
+        return t128 <= cus ? wave_split_or(c, M, N, K, cus) : c;
     }
     // Work of the busiest CU: rounds times tile area times K plus what a tile
     // costs beside its K loop (as that many K), over the tiling's rate.  Fitted

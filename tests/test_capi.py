@@ -254,6 +254,12 @@ def test_two_k_groups_where_tiles_fit_the_cus(M, N, K, k2):
     assert h3mi.config_for(M, N, K) == ("d_bm128_bn128_bk128_s2_g8_w2x2_sw_k2" if k2 else "d_bm128_bn128_bk128_s2_g4_o2")
 
 
+@pytest.mark.parametrize("M,N,K", [(671, 6312, 4992), (7714, 616, 10624), (871, 4816, 5248), (395, 11632, 10880), (316, 11200, 4736)])
+def test_no_wave_split_tiles_past_one_small_tile_per_cu(M, N, K):
+    import h3mi
+    assert h3mi.config_for(M, N, K) == "d_bm128_bn128_bk128_s2_g4_o2"
+
+
 @pytest.mark.parametrize("M,N,K,wide", [(2400, 9216, 1536, True), (1536, 13824, 768, True), (4096, 5376, 768, True),
                                         (4096, 5376, 384, False), (768, 28672, 384, False)])
 def test_256x384_tiles_on_small_grids_by_k(M, N, K, wide):
