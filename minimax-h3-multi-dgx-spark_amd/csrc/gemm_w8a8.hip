@@ -1028,11 +1028,15 @@ double predicted_us(int config, int64_t M, int64_t N, int64_t K, int64_t cus) {
 
 // The wave-split tiling with the least predicted time, or `other` if that is
 // faster still.  A tile with a whole 16-row block past M is left out: it
-// multiplies and sums blocks of zeros.
+// multiplies and sums blocks of zeros.  With K below 1536 the model has the
+// wave-split tiles about 20% too fast (their hand-off is half of such a call), so
+// they must be predicted that much ahead: of 200 outputs with K up to 1280 the 14
+// that were 3-24% behind `other` (55 x 20352 x 640 9.9 against 8.0 us, 1204 x 896 x
+// 768 9.2 against 8.0) all had less of a lead.
 int wave_split_or(int other, int64_t M, int64_t N, int64_t K, int64_t cus) {
     static const int first = config_index("k_bm16_bn16_w4_s2");
     int best = other;
-    double t = predicted_us(other, M, N, K, cus);
+    double t = predicted_us(other, M, N, K, cus) * (K < 1536 ? 0.82 : 1.0);
     for (int i = first; i < kNumConfigs; ++i) {
         if (kConfigs[i].bm > 16 && kConfigs[i].bm - 16 >= M) continue;
         const double ti = predicted_us(i, M, N, K, cus);

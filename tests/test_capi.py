@@ -260,6 +260,14 @@ def test_no_wave_split_tiles_past_one_small_tile_per_cu(M, N, K):
     assert h3mi.config_for(M, N, K) == "d_bm128_bn128_bk128_s2_g4_o2"
 
 
+@pytest.mark.parametrize("M,N,K,split", [(55, 20352, 640, False), (1204, 896, 768, False), (172, 6776, 640, False),
+                                         (36, 14652, 768, False), (875, 376, 13952, True), (84, 7128, 896, True),
+                                         (549, 896, 384, True), (10, 17648, 512, True)])
+def test_wave_split_tiles_with_short_k(M, N, K, split):
+    import h3mi
+    assert h3mi.config_for(M, N, K).startswith("k_") == split
+
+
 @pytest.mark.parametrize("M,N,K,wide", [(2400, 9216, 1536, True), (1536, 13824, 768, True), (4096, 5376, 768, True),
                                         (4096, 5376, 384, False), (768, 28672, 384, False)])
 def test_256x384_tiles_on_small_grids_by_k(M, N, K, wide):
