@@ -971,6 +971,14 @@ int resident_per_cu(kernel_fn fn, int threads) {
     return n;
 }
 
+// Whether a configuration can run a call: K a multiple of its K step (split-K
+// tilings need K % 256 == 0), and, with one workgroup per tile, fewer than the
+// 2^32 threads that HIP takes in a launch (16x16 tiles reach them at 2^32 outputs).
+bool takes(const Config& c, int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    return K % c.kmul == 0 && (c.resident || tiles < (int64_t{1} << 32) / c.threads);
+}
+
 // Predicted time of a tiling on a grid that does not fill the chip several
 // times over, in us.  A CU runs ceil(tiles / CUs) workgroups one after the
 // other (or side by side at a shared rate); a workgroup takes `tile` plus, per
@@ -1054,10 +1062,10 @@ int wave_split_or(int other, int64_t M, int64_t N, int64_t K, int64_t cus) {
 // `sectors`: the output's rows start on 32-byte sectors (gemm_entry).
 int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
     {
-        // a forced configuration that cannot take this K (split-K tilings
-        // need K % 256 == 0) leaves the call to the heuristic
+        // a forced configuration that cannot take this call leaves it to the
+        // heuristic
         std::lock_guard<std::mutex> lk(g_cfg_mu);
-        if (g_forced >= 0 && K % kConfigs[g_forced].kmul == 0) return g_forced;
+        if (g_forced >= 0 && takes(kConfigs[g_forced], M, N, K)) return g_forced;
     }
     static const int wide = config_index("d_bm256_bn384_bk128_s2_g8_w8m_l4_a1_sw_res");
     static const int wide4 = config_index("d_bm256_bn384_bk128_s2_g4_w8m_l4_a1_sw_res");

@@ -21,8 +21,8 @@ its wider candidate list does (:11-21, 69-71): the first call per
 keeps the fastest.  Every configuration gives the same bytes, so tuning never
 changes a result.  A forced configuration (set_config, the pin, a tuned call)
 is process-wide: a GEMM another thread launches meanwhile runs under it, which
-can change its speed, never its bytes (a configuration whose K multiple does not
-divide the call's K is ignored for that call).
+can change its speed, never its bytes (a configuration that cannot run a call,
+by its K multiple or by the size of the launch, is ignored for that call).
 """
 import ctypes
 import logging

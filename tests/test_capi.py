@@ -268,6 +268,18 @@ def test_wave_split_tiles_with_short_k(M, N, K, split):
     assert h3mi.config_for(M, N, K).startswith("k_") == split
 
 
+def test_forced_configuration_a_launch_cannot_hold_is_ignored():
+    """One workgroup of 256 threads per 16x16 tile: 2^32 outputs would be 2^32 threads."""
+    import h3mi
+    auto = h3mi.config_for(1 << 17, 1 << 15, 256)
+    try:
+        h3mi.set_config("k_bm16_bn16_w4_s2")
+        assert h3mi.config_for((1 << 17) - 16, 1 << 15, 256) == "k_bm16_bn16_w4_s2"
+        assert h3mi.config_for(1 << 17, 1 << 15, 256) == auto
+    finally:
+        h3mi.set_config("auto")
+
+
 @pytest.mark.parametrize("M,N,K,wide", [(2400, 9216, 1536, True), (1536, 13824, 768, True), (4096, 5376, 768, True),
                                         (4096, 5376, 384, False), (768, 28672, 384, False)])
 def test_256x384_tiles_on_small_grids_by_k(M, N, K, wide):
