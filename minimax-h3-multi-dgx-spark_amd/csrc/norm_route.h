@@ -9,7 +9,8 @@
 namespace h3mi {
 
 // A launch of S workgroups of 256 threads must stay below 2^32 threads, which
-// HIP refuses; the streams' grids do not grow with S.
+// HIP refuses; the streams' grids do not grow with S, so they take longer calls
+// at every width and number of table rows.
 inline bool rows_launchable(int64_t S) { return S < (int64_t{1} << 24); }
 
 // The norms.  Lines between the two routes, each measured on both sides over N

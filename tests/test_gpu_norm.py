@@ -138,16 +138,13 @@ def test_rejects_aliasing_and_bad_shapes():
         h.gate_(x6, x6.clone(), torch.ones(1, 66, device="cuda", dtype=torch.bfloat16), ridx)
 
 
-# Persistent row-stream kernels (N <= 8192, product order): rows handled by one
-# wave span several strides, tables staged in LDS (one table row), mixed table
-# rows (two segments: the majority row staged, the rest from global memory),
-# random table rows, the widest stream row and the first row past it, fewer
-# rows than one workgroup has waves, and more than 256 rows per workgroup
-# (the table-row count takes several steps), with one table row and with two
-# segments.  gate_norm_mod_ runs one row per workgroup where N is a multiple of
-# 1024 (5120, 8192, 1024, 2048 here) or 1024 IT + 256 (5376, 1280, 7424: the
-# last 256 elements' elementwise work one element per thread), and the row
-# stream otherwise.
+# Rows of N <= 8192 in the product order: one table row, two segments of unequal
+# length, random table rows, the widest row that the row streams and the
+# one-row-per-workgroup kernels take and the first past it, a row tail, fewer
+# rows than one workgroup of a stream has waves, and 70001 rows.  Most of these
+# calls are few enough rows to run one row per workgroup; 70001 rows over one
+# table row run the persistent streams (norm_mod).  The streams are held against
+# the one-row-per-workgroup kernels in test_gpu_norm_routes.py.
 STREAM_CASES = [
     ("uniform", 3001, 5120, 1),
     ("few", 5, 5120, 2),
@@ -213,9 +210,9 @@ def test_stream_gate_bitexact(kind, S, N, R):
 
 @pytest.mark.parametrize("N,R", [(5120, 2), (1028, 2), (5120, 1), (5376, 1)])
 def test_stream_out_of_range_rows_untouched(N, R):
-    """Rows whose table index is out of range are left unwritten (h and x),
-    both when they are a workgroup's majority and when they are not, with one
-    table row (R = 1) as with two."""
+    """Rows whose table index is out of range are left unwritten (h and x), with
+    one table row (R = 1) as with two: one row per workgroup, and at N = 1028 one
+    wave per row.  (The streams: test_gpu_norm_routes.py.)"""
     h = _h3mi()
     S = 2100
     x, w, s1, sh, g, o, ridx = norm_inputs(S, N, R, seed=N + R, stress=False)

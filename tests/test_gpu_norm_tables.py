@@ -1,7 +1,6 @@
 """The fused norms with many adaLN table rows: 257 rows of s1 / shift / gate and
-a random row per token, so that almost every row reads its table row through
-the range-checked global loads rather than the workgroup's row staged in LDS,
-at widths on the row-stream, hidden-5376 and widest stream paths."""
+a random row per token, each read through range-checked global loads (999 rows
+run one row per workgroup), at narrow, hidden-5120, hidden-5376 and widest rows."""
 import numpy as np
 import pytest
 import torch

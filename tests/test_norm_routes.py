@@ -62,3 +62,11 @@ def test_no_workgroup_per_row_past_the_launch_limit(routes, op, N, R):
 ])
 def test_route_of_the_faster_side(routes, op, S, N, R, rows):
     assert routes(op, S, N, R) == rows
+
+
+def test_the_gpu_tests_of_the_streams_reach_them(routes):
+    import test_gpu_norm_routes as t
+    for S, N, R, ops in t.STREAMS:
+        for op in ops:
+            assert not routes(op, S, N, R), (op, S, N, R)
+            assert routes(op, 700, N, R)  # the calls they are held against
