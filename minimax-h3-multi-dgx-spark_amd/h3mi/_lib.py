@@ -1,12 +1,15 @@
 """ctypes binding of libh3mi.so (the C ABI declared in include/h3mi.h).
 
-The library is loaded from this package directory.  There is no fallback: if
-the library is missing or does not export the ABI, importing the callers
-fails loudly (build it with `make -C minimax-h3-multi-dgx-spark_amd` or
-the repository's `build()` entry point).
+The library is loaded from this package directory, and with it _fast, the Python
+extension over it.  There is no fallback: if either is missing, does not export
+the ABI or was built for another python or torch, importing the callers
+fails loudly (build both with `make -C minimax-h3-multi-dgx-spark_amd` or
+the repository's `build()` entry point, under the interpreter that will run
+them).
 """
 import ctypes
 import os
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libh3mi.so")
@@ -79,7 +82,11 @@ lib = _load()
 
 import torch  # noqa: E402,F401  (its libraries, which _fast links)
 
-from . import _fast  # noqa: E402  (the common calls in native code; like libh3mi.so, built by the Makefile)
+try:
+    from . import _fast  # noqa: E402  (the common calls in native code)
+except ImportError as e:
+    raise ImportError(f"h3mi/_fast is not built for this python and torch ({e}); run "
+                      f"`make -C {os.path.dirname(_HERE)} PYTHON={sys.executable}`") from e
 
 _fast.set_error(H3miError)
 

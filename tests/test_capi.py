@@ -309,3 +309,20 @@ def test_buffer_probe_argument_errors():
     for args, code, msg in cases:
         st, m = _err(L.h3mi_debug_buffer_lds_load(*args, None))
         assert st == code and msg in m, (args, st, m)
+
+
+def test_import_without_the_extension_says_how_to_build_it(tmp_path):
+    """libh3mi.so there, _fast.so missing: an ImportError that names the make command, as for the library itself."""
+    import shutil
+    import subprocess
+    import sys
+    pkg = tmp_path / "h3mi"
+    pkg.mkdir()
+    src = os.path.dirname(LIB)
+    for f in os.listdir(src):
+        if f.endswith(".py"):
+            shutil.copy(os.path.join(src, f), pkg / f)
+    os.symlink(LIB, pkg / "libh3mi.so")
+    r = subprocess.run([sys.executable, "-c", "import h3mi"], cwd=tmp_path, capture_output=True, text=True, timeout=300,
+                       env={**os.environ, "PYTHONPATH": str(tmp_path)})
+    assert r.returncode != 0 and "ImportError" in r.stderr and "make -C" in r.stderr and "_fast" in r.stderr, r.stderr
