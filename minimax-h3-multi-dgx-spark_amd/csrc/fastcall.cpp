@@ -4,14 +4,15 @@
 // A call from Python through ctypes costs 10-14 us of host time (tensor checks,
 // allocation, the stream lookup, argument conversion), 27 for the two launches
 // of a W8A8 linear: more than the kernels of a short call.  Here the same checks,
-// allocations and launches take 3-6 us.
+// allocations and launches take 4-9 us.
 //
 // Every function returns None without doing anything unless its arguments are
 // what the Python function accepts in its plain form: exact torch tensors on one
-// GPU, with the types, shapes and strides checked here and no tensor mode or
-// transform active.  The Python function then runs its own checks, so every
-// other form, and every error, is decided there.  A nonzero status of the C ABI
-// raises the H3miError that the Python path raises.
+// GPU, with the types, shapes and strides checked here, none of them wrapped by a
+// transform, and no torch-function mode active.  The Python function then runs
+// its own checks, so every other form, and every error, is decided there.  A
+// dispatch mode sees the allocations of either path, and nothing else of them.
+// A nonzero status of the C ABI raises the H3miError that the Python path raises.
 #include <Python.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>

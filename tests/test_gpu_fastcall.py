@@ -101,7 +101,7 @@ def test_norms_and_rope(monkeypatch):
 
 
 def test_autograd_and_modes(monkeypatch):
-    """A call inside vmap, under a dispatch mode, on another stream."""
+    """A call inside vmap, under a dispatch mode, on another stream.  (Autograd: the next test.)"""
     import h3mi
     from torch.utils._python_dispatch import TorchDispatchMode
     x, w, ws, _ = (t.cuda() for t in gemm_inputs(16, 64, 256, seed=1))
@@ -125,3 +125,35 @@ def test_autograd_and_modes(monkeypatch):
         y = h3mi.w8a8_linear(x, w, ws)
     s.synchronize()
     assert torch.equal(y, ref)
+
+
+def test_requires_grad_and_function_modes(monkeypatch):
+    """Arguments that require grad give the same bytes, without a graph, on both
+    paths; under a torch-function mode the call is Python's, and the mode sees it."""
+    import h3mi
+    from torch.overrides import TorchFunctionMode
+    x, w, ws, bias = (t.cuda() for t in gemm_inputs(16, 64, 256, seed=2))
+    ref = h3mi.w8a8_linear(x, w, ws, bias)
+    xg, wsg = x.clone().requires_grad_(), ws.clone().requires_grad_()
+    a, b = _both(monkeypatch, lambda h: h.w8a8_linear(xg, w, wsg, bias))
+    assert _same(a, b) and torch.equal(a, ref) and not a.requires_grad
+    n = norm_inputs(9, 264, 2, seed=4, stress=False)
+    nx, nw, s1, sh, g, o, ridx = (t.cuda() for t in n)
+    a, b = _both(monkeypatch, lambda h: h.norm_mod(nx.clone().requires_grad_(), nw, 1e-6, ridx, s1, sh))
+    assert _same(a, b) and not a.requires_grad
+    with torch.no_grad():
+        a, b = _both(monkeypatch, lambda h: [h.gate_(nx.clone().requires_grad_(), o, g, ridx)])
+    assert _same(a, b)
+
+    class Seen(TorchFunctionMode):
+        n = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            Seen.n += 1
+            return func(*args, **(kwargs or {}))
+
+    with Seen():
+        assert torch.equal(h3mi.w8a8_linear(x, w, ws, bias), ref)
+        before = Seen.n
+        h3mi.norm_mod(nx, nw, 1e-6, ridx, s1, sh)
+    assert before > 0 and Seen.n > before
