@@ -83,7 +83,7 @@ int h3mi_w8a8_gemm_i32(const int8_t* xq, const int8_t* w, int32_t* acc,
                        int64_t ldx, int64_t ldw, int64_t ldc, void* stream);
 
 /* Tile configuration the GEMM uses for (M, N, K) with a contiguous output (one
- * whose rows start off 32-byte sectors may run another): the counterpart of the
+ * whose rows start off 64-byte half lines may run another): the counterpart of the
  * autotuner's best_config (comfyui_nodes/h3-linear-fast/int8_gemm_triton.py:32,
  * read at tests/test_triton_gemm.py:24).  Writes a NUL-terminated name. */
 int h3mi_w8a8_config(int64_t M, int64_t N, int64_t K, char* buf, int64_t buflen);

@@ -1059,8 +1059,8 @@ int wave_split_or(int other, int64_t M, int64_t N, int64_t K, int64_t cus) {
 // the smaller grids, one of the 128x128, 128x192 or larger tiles is picked by
 // whole rounds over the CUs times tile area and then weighed against the
 // wave-split tilings by predicted time.
-// `sectors`: the output's rows start on 32-byte sectors (gemm_entry).
-int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
+// `halves`: the output's rows start on 64-byte half lines (gemm_entry).
+int pick_config(int64_t M, int64_t N, int64_t K, bool halves) {
     {
         // a forced configuration that cannot take this call leaves it to the
         // heuristic
@@ -1085,9 +1085,9 @@ int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
     // work per CU: N = 15360 and 5120); with a ragged last column (N = 5376)
     // they measured 3-4% slower than 320x256, so they are offered only then.
     const bool n320 = N % 320 == 0;
-    // 256x384 tiles are offered when output rows start on sectors: their epilogue
+    // 256x384 tiles are offered when output rows start on half lines: their epilogue
     // has no room for the cached stores that other rows want (32768 x 9000 x 5120
-    // 1300 against 1208 us, x 768 515 against 306).  On sectors off 128-byte
+    // 1300 against 1208 us, x 768 515 against 306).  On half lines off whole
     // lines they stay ahead where the rounds say so (16000 x 5408 x 5120 364
     // against 374, 16000 x 10272 x 3072 421 against 437).
     const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
@@ -1118,7 +1118,7 @@ int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
         // 116, 4096 x 5376 x 14336 260 against 327, 2400 x 9216 x 1536 39 against 44,
         // x 768 26.8 against 28.7; at K = 384 its epilogue weighs more (4096 x 5376
         // 20.3 against 19.9).
-        const double c384 = sectors && K >= 768 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
+        const double c384 = halves && K >= 768 ? rounds(256, 384) * 256.0 * 384.0 / (1.5 * 1.03) : 1e300;
         const double ck2 = K % 256 == 0 ? rounds(128, 192) * 128.0 * 192.0 / 0.88 : 1e300;
         int c = c256 < c128 ? big : small;
         if (ck2 < c256 && ck2 < c128) c = split;
@@ -1143,7 +1143,7 @@ int pick_config(int64_t M, int64_t N, int64_t K, bool sectors) {
     // areas alone, which sent short K to 256x384 tiles (10000 x 13824 x 384 110
     // against 88 us, 32768 x 13824 x 768 439 against 383).
     const double w256 = rounds(256, 256) * 256.0 * 256.0 * (K + 554);
-    const double w384 = sectors ? rounds(256, 384) * 256.0 * 384.0 * (K + 820) / 1.07 : 1e300;
+    const double w384 = halves ? rounds(256, 384) * 256.0 * 384.0 * (K + 820) / 1.07 : 1e300;
     const double w320 = rounds(320, 256) * 320.0 * 256.0 * (K + 541);
     const double w320n = n320 ? rounds(256, 320) * 256.0 * 320.0 * (K + 640) / 1.024 : 1e300;
     if (w320n < w256 && w320n < w384 && w320n < w320) return flat;
@@ -1181,21 +1181,22 @@ int gemm_entry(const int8_t* xq, const int8_t* w, const float* xs, const float* 
     const size_t ob = static_cast<size_t>(M) * ldo * (OUT_I32 ? 4 : 2);
     if (overlap(out, ob, xq, static_cast<size_t>(M) * ldx) || overlap(out, ob, w, static_cast<size_t>(N) * ldw))
         return fail(H3MI_EALIAS, "%s: out overlaps an input", name);
-    const bool sectors = ldo % 16 == 0 && aligned(out, 32);
-    const Config& c = kConfigs[pick_config(M, N, K, sectors)];
+    const bool halves = ldo % 32 == 0 && aligned(out, 64);
+    const Config& c = kConfigs[pick_config(M, N, K, halves)];
     const int tiles_m = static_cast<int>((M + c.bm - 1) / c.bm), tiles_n = static_cast<int>((N + c.bn - 1) / c.bn);
     const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
     if (tiles > 0x7FFFFFFF) return fail(H3MI_EINVAL, "%s: too many tiles", name);
-    // Output rows that start off 32-byte sectors (N = 9000) are stored through the
-    // cache once the output is past 16 MiB: a slab's segment of a row ends inside
-    // sectors whose other parts the neighbouring slabs write, and non-temporal
-    // stores send each part to memory by itself; the L2 joins them (256x256 tiles,
-    // 10000 x 9000 x 384 110 -> 72 us, 11504 x 1192 x 512 19.8 -> 15.5, 2182 x 12856
-    // x 3072 93 -> 85).  Over 140 shapes: rows on sectors, smaller outputs and
-    // 128x128 tiles were the same or up to 10% faster with non-temporal stores
-    // (2961 x 2336 x 1280 14.3 against 15.8, 8903 x 648 x 896 11.7 against 12.7).
+    // Output rows that start off 64-byte half lines (N = 9000) are stored through
+    // the cache once the output is past 16 MiB: a slab's segment of a row ends
+    // inside half lines whose other parts the neighbouring slabs write, and
+    // non-temporal stores send each part to memory by itself; the L2 joins them
+    // (256x256 tiles, 10000 x 9000 x 384 110 -> 72 us, 11504 x 1192 x 512 19.8 -> 15.5,
+    // 3000 x 10224 x 384 36 -> 26).  Rows on half lines, smaller outputs and 128x128
+    // tiles were the same or up to 14% faster with non-temporal stores (4149 x
+    // 2656 x 384 12.0 against 13.9, 2961 x 2336 x 1280 14.3 against 15.8, 8903 x 648 x
+    // 896 11.7 against 12.7).
     // A kernel of its own, so that the others' epilogue stays free of it.
-    const bool cached = c.bf16_cached && !sectors && M * N > int64_t{8} << 20;
+    const bool cached = c.bf16_cached && !halves && M * N > int64_t{8} << 20;
     const kernel_fn fn = OUT_I32 ? c.i32_kernel : cached ? c.bf16_cached : c.bf16_kernel;
     int64_t grid = tiles;
     if (c.resident) {
@@ -1271,7 +1272,7 @@ extern "C" int h3mi_w8a8_gemm_i32(const int8_t* xq, const int8_t* w, int32_t* ac
 
 extern "C" int h3mi_w8a8_config(int64_t M, int64_t N, int64_t K, char* buf, int64_t buflen) {
     if (!buf || buflen <= 0) return fail(H3MI_EINVAL, "w8a8_config: no buffer");
-    const char* nm = kConfigs[pick_config(M, N, K, N % 16 == 0)].name;  // a contiguous, aligned output
+    const char* nm = kConfigs[pick_config(M, N, K, N % 32 == 0)].name;  // a contiguous, aligned output
     strncpy(buf, nm, static_cast<size_t>(buflen - 1));
     buf[buflen - 1] = '\0';
     return ok();

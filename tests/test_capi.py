@@ -288,8 +288,8 @@ def test_256x384_tiles_on_small_grids_by_k(M, N, K, wide):
     assert h3mi.config_for(M, N, K).startswith("d_bm256_bn384") == wide
 
 
-@pytest.mark.parametrize("N,wide", [(10304, True), (10272, True), (10256, True), (10280, False), (10276, False)])
-def test_256x384_tiles_need_output_rows_on_sectors(N, wide):
+@pytest.mark.parametrize("N,wide", [(10304, True), (10272, True), (10256, False), (10280, False), (10276, False)])
+def test_256x384_tiles_need_output_rows_on_half_lines(N, wide):
     import h3mi
     assert h3mi.config_for(16000, N, 5120).startswith("d_bm256_bn384") == wide
 

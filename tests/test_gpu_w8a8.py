@@ -374,11 +374,11 @@ def test_allcfg_autotune_picks_a_config_and_keeps_the_bytes(monkeypatch):
     assert h3mi.config_for(M, N, K) == h3mi.config_for(M, N, K)  # the heuristic is restored after each call
 
 
-@pytest.mark.parametrize("N,ldo,off", [(1000, 1000, 0), (1000, 1028, 0), (1024, 1024, 4), (968, 1024, 0), (1024, 1040, 16)])
-def test_output_rows_off_sectors(N, ldo, off):
-    """Output rows that start off 32-byte sectors (their length, their stride or
+@pytest.mark.parametrize("N,ldo,off", [(1000, 1000, 0), (1000, 1028, 0), (1024, 1024, 4), (968, 1024, 0), (1024, 1040, 16), (1024, 1056, 32)])
+def test_output_rows_off_half_lines(N, ldo, off):
+    """Output rows that start off 64-byte half lines (their length, their stride or
     the first row's address), in an output past the 16 MiB from which they are
-    stored through the cache, and rows on sectors: every configuration writes the
+    stored through the cache, and rows on them: every configuration writes the
     exact epilogue's bytes, whole tiles and edges, and nothing beside them."""
     h = _h3mi()
     from h3mi._lib import check, lib, ptr, stream_of
@@ -391,7 +391,7 @@ def test_output_rows_off_sectors(N, ldo, off):
     want = {False: plain.to(torch.bfloat16), True: (plain + bias.float()).to(torch.bfloat16)}
     try:
         for name in h.list_configs():
-            print(f"[rows off sectors] {name} N={N} ldo={ldo} off={off}", flush=True)
+            print(f"[rows off half lines] {name} N={N} ldo={ldo} off={off}", flush=True)
             h.set_config(name)
             for b in (False, True):
                 buf = torch.full((M * ldo + off + 64,), 7, dtype=torch.bfloat16, device="cuda")
