@@ -596,7 +596,7 @@ def bench_norms(torch, h3mi, args):
         res[name] = {"ms": ms, "bytes": nbytes, "gbs": gbs, "frac": gbs / PEAK_HBM_GBS, "unfused_ms": ums}
         log(f"[bench] {name}: {ms * 1e3:.1f} us, {gbs:.0f} GB/s ({100 * gbs / PEAK_HBM_GBS:.1f}% of 8 TB/s); "
             f"norm then quantizer: {ums * 1e3:.1f} us")
-    # copy bandwidth the box achieves (context for the fractions above)
+    # copy bandwidth this card achieves (context for the fractions above)
     src = torch.empty(S * N * 2, dtype=torch.uint8, device=dev)
     dst = torch.empty_like(src)
     for _ in range(3):
@@ -861,7 +861,7 @@ def bench_h3(torch, h3mi, args):
     log(f"[bench] h3 rms_rope_split_half_ q,k [{S}, {H}, {D}]: {ms * 1e3:.1f} us, {nb / ms / 1e6:.0f} GB/s "
         f"({100 * nb / ms / 1e6 / PEAK_HBM_GBS:.1f}%)")
     del qkv
-    # a device copy of COPY_BYTES: the box's copy rate, and the reference launch the rocprof traffic summary
+    # a device copy of COPY_BYTES: this card's copy rate, and the reference launch the rocprof traffic summary
     # calibrates FETCH_SIZE / WRITE_SIZE against
     src = torch.empty(int(COPY_BYTES), dtype=torch.uint8, device=dev)
     dst = torch.empty_like(src)

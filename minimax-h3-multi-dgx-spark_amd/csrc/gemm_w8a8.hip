@@ -987,7 +987,7 @@ bool takes(const Config& c, int64_t M, int64_t N, int64_t K) {
 // 5.3 TB/s.  The constants are least-squares fits to 300 measured shapes (M 1 to
 // 4799, N 384 to 28672, K 384 to 14336; relative error 8-11%, larger only where
 // a tiling is far from the best).  Over these shapes the rule below picks a
-// tiling 3% slower than the fastest of them on average, against 45% for the
+// tiling 2% slower than the fastest of them on average, against 41% for the
 // rule over the 128x128 and larger tiles alone.
 struct Cost {
     const char* name;
